@@ -139,6 +139,37 @@ struct HipError : std::runtime_error {
 
 inline unsigned ceil_div(size_t a, size_t b) { return (unsigned)((a + b - 1) / b); }
 
+// How many z ranges of its block each (tile, block) of a stage launch is
+// split into.  A workgroup marches its column plane by plane, so a launch of
+// few tiles leaves compute units idle for the whole march; ranges fill them
+// at the price of the lead-in planes each range repeats (about two planes'
+// worth of work).  With k workgroups to a compute unit, run in r rounds of at
+// most per_cu, an iteration of the march costs `lat` (its barriers and loads,
+// once a round, however many workgroups overlap there) plus one share per
+// workgroup, so the launch takes about (n_z / kz + 2) (lat r + k).  `lat` is
+// fitted to sweeps of kz over 30 meshes of 32^3 to 256^3 cells: 0.5 for the
+// FP64 MHD kernel (one workgroup nearly saturates a compute unit), 1.5 for
+// the mixed MHD kernels, 2.5 for the hydro kernel.  Measured, ms per cycle at
+// kz = 1 and at the rule's: 32^3 MHD FP64 in 16^3 blocks 0.392 -> 0.107,
+// 64^3 MHD FP64 in one block 1.39 -> 0.25, 64^3 MHD mixed in 32^3 blocks
+// 0.36 -> 0.13, 128^3 hydro mixed in 32^3 blocks 0.32 -> 0.24; from 128^3
+// (FP64 MHD) or 256^3 cells on the tiles fill the GPU and kz stays 1.
+constexpr double kLatMhd64 = 0.5, kLatMhdMixed = 1.5, kLatHydro = 2.5;
+
+unsigned z_ranges(size_t wgs, int ncu, int per_cu, int nz, double lat) {
+    unsigned best = 1;
+    double cost = 0;
+    for (int kz = 1; kz <= std::max(1, nz / 2); ++kz) {
+        const double k = (double)ceil_div(wgs * kz, ncu), r = (double)ceil_div((size_t)k, per_cu);
+        const double t = ((double)ceil_div(nz, kz) + 2) * (lat * r + k);
+        if (kz == 1 || t < cost) {
+            cost = t;
+            best = (unsigned)kz;
+        }
+    }
+    return best;
+}
+
 // graph replays between host checks of the stop rule in kr_advance
 constexpr int kAdvanceChunk = 64;
 
@@ -184,7 +215,9 @@ struct kr_ctx {
     bool mx_list = false;           // k_sweep_mx walks a device work list (ensembles)
     int4 *d_items = nullptr;        // its items (block, tile, z0, z1) and their count
     int *d_nitems = nullptr;
-    int slots[16] = {0};            // resident workgroups on the GPU per variant (0: not asked yet)
+    int ncu = 0;                    // compute units (0: not asked yet)
+    int per_cu[16] = {0};           // resident workgroups per compute unit by variant, 15 the
+                                    // producer forms (0: not asked yet)
     std::vector<int> candidates;    // variants the autotuner times
     int tune_next = 0;              // next candidate to time
     bool tuned = false;
@@ -764,15 +797,37 @@ struct Launcher {
         evs.push_back({kind, {a, b}});
     }
 
+    // Workgroups of a kernel that one compute unit holds, asked once.
+    int resident(int variant, const void *fn, int threads) {
+        if (c->ncu == 0) {
+            int dev = 0;
+            KR_HIP(hipGetDevice(&dev));
+            KR_HIP(hipDeviceGetAttribute(&c->ncu, hipDeviceAttributeMultiprocessorCount, dev));
+        }
+        int &n = c->per_cu[variant];
+        if (n == 0) {
+            KR_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, fn, threads, 0));
+            n = std::max(1, n);
+        }
+        return n;
+    }
+    // z ranges of a launch of `fn` on nt tiles of nb blocks
+    template <class K> unsigned ranges(K fn, int variant, int threads, unsigned nt, unsigned nb, double lat) {
+        const int per = resident(variant, reinterpret_cast<const void *>(fn), threads);
+        return z_ranges((size_t)nt * nb, c->ncu, per, c->n[2], lat);
+    }
     template <class FT, int TX, int TY, int NT, int W, int PROD = 0>
     void sweep_t(const MeshView<FT> &m, int step, unsigned nb) {
         const unsigned nt = (unsigned)((c->n[0] / TX) * (c->n[1] / TY));
+        auto go = [&](auto fn) {
+            const unsigned kz = ranges(fn, PROD ? 15 : c->variant, NT, nt, nb,
+                                       std::is_same_v<FT, double> ? kLatMhd64 : kLatMhdMixed);
+            hipLaunchKernelGGL(fn, dim3(nt, nb, kz), dim3(NT), 0, c->stream, m, step);
+        };
         if (c->npfill)                      // physical sides (one-level meshes only)
-            hipLaunchKernelGGL((k_sweep<FT, TX, TY, NT, W, PROD, true>), dim3(nt, nb), dim3(NT), 0,
-                               c->stream, m, step);
+            go(k_sweep<FT, TX, TY, NT, W, PROD, true>);
         else
-            hipLaunchKernelGGL((k_sweep<FT, TX, TY, NT, W, PROD, false>), dim3(nt, nb), dim3(NT), 0,
-                               c->stream, m, step);
+            go(k_sweep<FT, TX, TY, NT, W, PROD, false>);
     }
     // fluxes and edge EMFs of the listed blocks into F / EE (no update)
     template <class FT> void sweep_prod(const MeshView<FT> &m, int step, unsigned nb) {
@@ -788,8 +843,9 @@ struct Launcher {
     template <class FT, int TX, int TY, int NT>
     void sweep_hyd_t(const MeshView<FT> &m, int step, unsigned nb) {
         const unsigned nt = (unsigned)((c->n[0] / TX) * (c->n[1] / TY));
-        hipLaunchKernelGGL((k_sweep_hyd<FT, TX, TY, NT>), dim3(nt, nb), dim3(NT), 0, c->stream, m,
-                           step);
+        const auto fn = k_sweep_hyd<FT, TX, TY, NT>;
+        const unsigned kz = ranges(fn, c->variant, NT, nt, nb, kLatHydro);
+        hipLaunchKernelGGL(fn, dim3(nt, nb, kz), dim3(NT), 0, c->stream, m, step);
     }
     // hydro: the one-wave-per-SIMD-minimum variants of the tile table
     template <class FT> void sweep_hyd(const MeshView<FT> &m, int step, int variant, unsigned nb) {
@@ -831,24 +887,21 @@ struct Launcher {
     void sweep_mx_t(const MeshView<float> &m, int step, unsigned nb) {
         const unsigned nt = (unsigned)((c->n[0] / TX) * (c->n[1] / TY));
         if (!c->mx_list) {
-            hipLaunchKernelGGL((k_sweep_mx<TX, TY, NT, false>), dim3(nt, nb), dim3(NT), 0, c->stream,
-                               m, step, (const int4 *)nullptr, (const int *)nullptr);
+            const auto fr = k_sweep_mx<TX, TY, NT, MX_RANGES>;
+            const unsigned kz = ranges(fr, c->variant, NT, nt, nb, kLatMhdMixed);
+            const auto fn = kz > 1 ? fr : k_sweep_mx<TX, TY, NT, MX_GRID>;
+            hipLaunchKernelGGL(fn, dim3(nt, nb, kz), dim3(NT), 0, c->stream, m, step,
+                               (const int4 *)nullptr, (const int *)nullptr);
             return;
         }
-        int &slots = c->slots[c->variant & 15];
-        if (slots == 0) {
-            int dev = 0, ncu = 0, per_cu = 0;
-            KR_HIP(hipGetDevice(&dev));
-            KR_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-            KR_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                &per_cu, reinterpret_cast<const void *>(k_sweep_mx<TX, TY, NT, true>), NT, 0));
-            slots = std::max(1, ncu * per_cu);
-        }
+        const int per = resident(
+            c->variant, reinterpret_cast<const void *>(k_sweep_mx<TX, TY, NT, MX_LIST>), NT);
+        const int slots = c->ncu * per;
         const unsigned lt = (unsigned)std::min<size_t>(1024, ceil_div((size_t)nb, 64) * 64);
         hipLaunchKernelGGL(k_sweep_list, dim3(1), dim3(lt), 0, c->stream, (const TimeState *)c->ts,
                            (const BlockGeo *)c->geo, (int)nb, (int)nt, c->n[2], slots, c->d_items,
                            c->d_nitems);
-        hipLaunchKernelGGL((k_sweep_mx<TX, TY, NT, true>), dim3(slots), dim3(NT), 0, c->stream, m,
+        hipLaunchKernelGGL((k_sweep_mx<TX, TY, NT, MX_LIST>), dim3(slots), dim3(NT), 0, c->stream, m,
                            step, (const int4 *)c->d_items, (const int *)c->d_nitems);
     }
 

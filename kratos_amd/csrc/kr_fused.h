@@ -59,6 +59,16 @@ struct TileShape {
     }
 };
 
+// Planes [z0, z1) of the block that this workgroup of a grid launch owns:
+// range blockIdx.z of gridDim.z.  A range repeats the march's lead-in planes
+// z0 - 2 .. z0 and solves the faces and edges at its ends as the neighbouring
+// range does, from the same inputs through the same code, and stores only its
+// own cells and faces, so a split changes no result.
+__device__ __forceinline__ void z_range(int nz, int &z0, int &z1) {
+    z0 = (int)blockIdx.z * nz / (int)gridDim.z;
+    z1 = ((int)blockIdx.z + 1) * nz / (int)gridDim.z;
+}
+
 __device__ __forceinline__ int ring3(int p) { return ((p % 3) + 3) % 3; }
 __device__ __forceinline__ int ring2(int p) { return (p + 4) & 1; }
 
@@ -178,6 +188,8 @@ k_sweep(MeshView<FT> m, int step) {
     const int ntx = m.n[0] / TX;
     const int x0 = (blockIdx.x % ntx) * TX, y0 = (blockIdx.x / ntx) * TY;
     const int nz = m.n[2];
+    int z0, z1;
+    z_range(nz, z0, z1);
     const bool xlast = x0 + TX == m.n[0], ylast = y0 + TY == m.n[1];
     const BlockGeo &g = m.geo[b];
     const double dt = m.ts[g.grp].dt_use * (step == 0 ? 1.0 : 0.5);
@@ -346,8 +358,8 @@ k_sweep(MeshView<FT> m, int step) {
     const double dt_dv = dt / g.vol;
 
 
-    issue_w(-2, ring3(-2));
-    for (int L = -2; L <= nz + 1; ++L) {
+    issue_w(z0 - 2, ring3(z0 - 2));
+    for (int L = z0 - 2; L <= z1 + 1; ++L) {
         // ------------------------------------------------ 1. plane L arrives
         __builtin_amdgcn_s_waitcnt(0);   // this wave's loads into the ring
         __syncthreads();                 // ... and every other wave's
@@ -355,7 +367,7 @@ k_sweep(MeshView<FT> m, int step) {
         const int P = L - 2;          // plane finished in this iteration
 
         // ------------------------------------------------ 2. fluxes
-        if (L >= 0) {
+        if (L >= z0) {
             const int p = L - 1;                 // plane of the in-plane faces / z face index
             const int s0 = ring3(p), sm = ring3(p - 1), sp = ring3(p + 1);
             const int fe = ring2(p);
@@ -383,7 +395,7 @@ k_sweep(MeshView<FT> m, int step) {
                         qLn[v] = q0 + (flat ? (FT)0 : t);
                     }
                 }
-                if (p >= 0 && p <= nz) {
+                if (p >= z0) {
                     FT wl[8], wr[8], flx[8];
 #pragma unroll
                     for (int v = 0; v < 8; ++v) {
@@ -407,15 +419,15 @@ k_sweep(MeshView<FT> m, int step) {
                     sFz[0][gz] = flx[RHO];
                     sFz[1][gz] = flx[BCC + 2];
                     sFz[2][gz] = -flx[BCC + 1];
-                    if (prod && zint) {
+                    if (prod && zint && (p < z1 || z1 == nz)) {
                         // the block's z face (x, y, p): hydro flux for the staged update
                         const int q3[3] = {x0 + cx_, y0 + cy_, p};
                         FT *F = m.F[2] + (size_t)b * 8 * m.nfa[2] + xidx(m.n, 2, q3);
 #pragma unroll
                         for (int v = 0; v < 5; ++v) F[(size_t)v * m.nfa[2]] = flx[v];
-                    } else if (zint) {
+                    } else if (!prod && zint) {
                         // z part of the cell finished now (plane p-1 = P)
-                        if (P >= 0) {
+                        if (P >= z0) {
                             const FT fa = F32 ? (FT)sGeo[3 + 2] : (FT)(g.sfc[2] * dt_dv);
                             const size_t cc = cidx(m.n, x0 + cx_, y0 + cy_, P);
                             double *Ut = m.U + ((size_t)b * 2 + (1 - step)) * 5 * nc + cc;
@@ -495,7 +507,7 @@ k_sweep(MeshView<FT> m, int step) {
                 if (prod) {
                     // a face of the block (not a transverse ghost line, not a
                     // ghost plane): hydro flux for the staged update
-                    if (!ghost_plane && (xf ? (fy >= 0 && fy < TY) : (fx >= 0 && fx < TX))) {
+                    if (p >= z0 && p < z1 && (xf ? (fy >= 0 && fy < TY) : (fx >= 0 && fx < TX))) {
                         const int q3[3] = {x0 + fx, y0 + fy, p};
                         FT *F = m.F[a] + (size_t)b * 8 * m.nfa[a] + xidx(m.n, a, q3);
                         F[(size_t)RHO * m.nfa[a]] = flx[RHO];
@@ -518,8 +530,10 @@ k_sweep(MeshView<FT> m, int step) {
         __syncthreads();
 
         // ------------------------------------------------ 3. EMFs
-        if (L >= 1) {
+        if (L >= z0 + 1) {
             const int p = L - 1;
+            // edges of z face p are stored by the range that owns the face
+            const bool own_p = p < z1 || z1 == nz;
             const int s0 = ring3(p), sm = ring3(p - 1);
             const int fe = ring2(p), fm = ring2(p - 1);
             auto ec = [&](int s, int x, int y, int c) -> FT {
@@ -565,7 +579,7 @@ k_sweep(MeshView<FT> m, int step) {
             };
             for (int it = tid; it < S::NEZ + S::NEX + S::NEY; it += NT) {
                 if (it < S::NEZ) {
-                    if (p >= nz) continue;
+                    if (p >= z1) continue;
                     const int x = it % (TX + 1), y = it / (TX + 1);
                     // ee_z on plane p: a1 = x, a2 = y
                     FT e = edge_emf<FT>(
@@ -590,7 +604,7 @@ k_sweep(MeshView<FT> m, int step) {
                         sFe[fe][0][S::fyi(x, y)], sFe[fm][0][S::fyi(x, y)]);
                     if (PHY && g.phy) e = bplane(0, x, y, e);
                     sEx[fe][S::exi(x, y)] = e;
-                    if (prod)
+                    if (prod && own_p)
                         m.EE[((size_t)b * 3 + 0) * m.nface + fidx(m.n, x0 + x, y0 + y, p)] = e;
                 } else {
                     const int k = it - S::NEZ - S::NEX;
@@ -604,7 +618,7 @@ k_sweep(MeshView<FT> m, int step) {
                         sFz[0][S::zg(x, y)], sFz[0][S::zg(x - 1, y)]);
                     if (PHY && g.phy) e = bplane(1, x, y, e);
                     sEy[fe][S::eyi(x, y)] = e;
-                    if (prod)
+                    if (prod && own_p)
                         m.EE[((size_t)b * 3 + 1) * m.nface + fidx(m.n, x0 + x, y0 + y, p)] = e;
                 }
             }
@@ -613,10 +627,10 @@ k_sweep(MeshView<FT> m, int step) {
 
         // plane L+1 into the slot of plane L-2, which phases 2 and 3 of this
         // iteration were the last to read; it lands while the update runs
-        if (L + 1 <= nz + 1) issue_w(L + 1, ring3(L + 1));
+        if (L + 1 <= z1 + 1) issue_w(L + 1, ring3(L + 1));
 
         // ------------------------------------------------ 4. update
-        if (!prod && L >= 1) {
+        if (!prod && L >= z0 + 1) {
             const int q = L - 1;                     // z face updated now
             const int fq = ring2(q), fpp = ring2(P);
             // Face-field update of one face (mhd/integrator/rk2.h:48-62): the
@@ -661,10 +675,10 @@ k_sweep(MeshView<FT> m, int step) {
             if (zint) {
                 const int x = cx_, y = cy_;
                 const FaceUpd uz = face_load(2, x, y, q);
-                const FaceUpd ux = face_load(0, x, y, P < 0 ? 0 : P);
-                const FaceUpd uy = face_load(1, x, y, P < 0 ? 0 : P);
+                const FaceUpd ux = face_load(0, x, y, P < z0 ? z0 : P);
+                const FaceUpd uy = face_load(1, x, y, P < z0 ? z0 : P);
                 // x + y partial of plane q (cells), finished next iteration
-                if (q < nz) {
+                if (q < z1) {
                     // conserved state of plane q, loaded here so that it is not
                     // live across the flux phase
                     const size_t c = cidx(m.n, x0 + x, y0 + y, q);
@@ -709,10 +723,12 @@ k_sweep(MeshView<FT> m, int step) {
 #pragma unroll
                     for (int v = 0; v < 5; ++v) part[v] = uu[v];
                 }
-                // z face q
-                face_store(uz, ct(sEx[fq][S::exi(x, y)], dx, sEy[fq][S::eyi(x, y)], dy,
-                                  sEy[fq][S::eyi(x + 1, y)], sEx[fq][S::exi(x, y + 1)], 2));
-                if (P >= 0) {
+                // z face q: the range's own faces, and the block's top face in
+                // the last range
+                if (q < z1 || z1 == nz)
+                    face_store(uz, ct(sEx[fq][S::exi(x, y)], dx, sEy[fq][S::eyi(x, y)], dy,
+                                      sEy[fq][S::eyi(x + 1, y)], sEx[fq][S::exi(x, y + 1)], 2));
+                if (P >= z0) {
                     // x face (x, y, P): a1 = y, a2 = z
                     face_store(ux, ct(sEy[fpp][S::eyi(x, y)], dy, sEz[fpp][S::ezi(x, y)], dz,
                                       sEz[fpp][S::ezi(x, y + 1)], sEy[fq][S::eyi(x, y)], 0));
@@ -721,13 +737,13 @@ k_sweep(MeshView<FT> m, int step) {
                                       sEx[fq][S::exi(x, y)], sEz[fpp][S::ezi(x + 1, y)], 1));
                 }
             }
-            if (P >= 0 && xedge) {
+            if (P >= z0 && xedge) {
                 const int x = TX, y = et;
                 set_face(0, x, y, P,
                          ct(sEy[fpp][S::eyi(x, y)], dy, sEz[fpp][S::ezi(x, y)], dz,
                             sEz[fpp][S::ezi(x, y + 1)], sEy[fq][S::eyi(x, y)], 0));
             }
-            if (P >= 0 && yedge) {
+            if (P >= z0 && yedge) {
                 const int x = et - TY, y = TY;
                 set_face(1, x, y, P,
                          ct(sEz[fpp][S::ezi(x, y)], dz, sEx[fpp][S::exi(x, y)], dx,

@@ -41,6 +41,8 @@ __global__ void __launch_bounds__(NT) k_sweep_hyd(MeshView<FT> m, int step) {
     const int ntx = m.n[0] / TX;
     const int x0 = (blockIdx.x % ntx) * TX, y0 = (blockIdx.x / ntx) * TY;
     const int nz = m.n[2];
+    int z0, z1;
+    z_range(nz, z0, z1);
     const BlockGeo &g = m.geo[b];
     const double dt = m.ts[g.grp].dt_use * (step == 0 ? 1.0 : 0.5);
     const FT gam = (FT)m.gamma;
@@ -115,15 +117,15 @@ __global__ void __launch_bounds__(NT) k_sweep_hyd(MeshView<FT> m, int step) {
     }
     const double dt_dv = dt / g.vol;
 
-    issue_w(-2, ring3(-2));
-    for (int L = -2; L <= nz + 1; ++L) {
+    issue_w(z0 - 2, ring3(z0 - 2));
+    for (int L = z0 - 2; L <= z1 + 1; ++L) {
         // ------------------------------------------------ 1. plane L arrives
         __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
         const int P = L - 2;
 
         // ------------------------------------------------ 2. fluxes
-        if (L >= 0) {
+        if (L >= z0) {
             const int p = L - 1;
             const int s0 = ring3(p), sm = ring3(p - 1), sp = ring3(p + 1);
             if (own) {
@@ -143,7 +145,7 @@ __global__ void __launch_bounds__(NT) k_sweep_hyd(MeshView<FT> m, int step) {
                         qLn[v] = q0 + (flat ? (FT)0 : t);
                     }
                 }
-                if (p >= 0 && p <= nz) {
+                if (p >= z0) {
                     FT wl[5], wr[5], flx[5];
 #pragma unroll
                     for (int v = 0; v < 5; ++v) {
@@ -157,7 +159,7 @@ __global__ void __launch_bounds__(NT) k_sweep_hyd(MeshView<FT> m, int step) {
                     else
                         hllc<FT>(flx, wl, wr, gam);
                     rot<1>(flx + MOM);
-                    if (P >= 0) {
+                    if (P >= z0) {
                         // z part of cell P: faces P (previous) and p = P + 1
                         const FT fa = F32 ? (FT)sFa[2] : (FT)(g.sfc[2] * dt_dv);
                         const size_t cc = cidx(m.n, x0 + cx, y0 + cy, P);
@@ -183,7 +185,7 @@ __global__ void __launch_bounds__(NT) k_sweep_hyd(MeshView<FT> m, int step) {
             }
             // in-plane faces of plane p; items start at the first lane past
             // the pencil lanes (a wave boundary) and wrap around
-            if (p >= 0 && p < nz)
+            if (p >= z0 && p < z1)
                 for (int it = tid - OWNP + (tid < OWNP ? NT : 0); it < NF; it += NT) {
                     if (it < 0) continue;
                     const bool xf = it < NFX;
@@ -232,11 +234,11 @@ __global__ void __launch_bounds__(NT) k_sweep_hyd(MeshView<FT> m, int step) {
 
         // plane L+1 into the slot of plane L-2, which phase 2 of this
         // iteration was the last to read; it lands while the update runs
-        if (L + 1 <= nz + 1) issue_w(L + 1, ring3(L + 1));
+        if (L + 1 <= z1 + 1) issue_w(L + 1, ring3(L + 1));
 
         // ------------------------------------------------ 3. x + y update of plane L-1
         const int q = L - 1;
-        if (own && q >= 0 && q < nz) {
+        if (own && q >= z0 && q < z1) {
             const size_t c = cidx(m.n, x0 + cx, y0 + cy, q);
             const double *Us = m.U + ((size_t)b * 2 + step) * 5 * nc + c;
             const double *Ut = m.U + ((size_t)b * 2 + (1 - step)) * 5 * nc + c;
