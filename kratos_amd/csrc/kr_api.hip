@@ -5,6 +5,7 @@
 #include "kr_fused.h"
 #include "kr_fused_hydro.h"
 #include "kr_smr.h"
+#include "kr_sweep64.h"
 #include "kr_sweep_mx.h"
 
 #include <hip/hip_runtime.h>
@@ -174,21 +175,35 @@ unsigned z_ranges(size_t wgs, int ncu, int per_cu, int nz, double lat) {
 constexpr int kAdvanceChunk = 64;
 
 // Fused stage-kernel variants: column tile, workgroup size, the minimum
-// waves per SIMD asked of the compiler (1 = no constraint), and the kernel:
-// k_sweep (mx = 0) or k_sweep_mx (mx = 1, the mixed form's kernel for MHD
-// meshes of one level without physical sides).  The autotuner times every
-// variant that fits the block shape and keeps the fastest; on a mesh that
-// k_sweep_mx serves it times only those (the two kernels round the FP32
-// fluxes differently, and the tuning cycles must leave the state any
-// single variant would), k_sweep's 4-wave builds being reachable there
-// only when kr_config.tile forces one.
-struct SweepVariant {
-    int tx, ty, nt, waves, mx;
+// waves per SIMD asked of the compiler (1 = no constraint), and the kernel.
+// The autotuner times the variants of the mesh's kernel that fit the block
+// shape and keeps the fastest.  A mesh runs one kernel throughout (k_sweep
+// and k_sweep_mx round the FP32 fluxes differently, and the tuning cycles
+// must leave the state any single variant would); on a mesh of k_sweep_mx,
+// k_sweep's 4-wave builds are reachable only when kr_config.tile forces one.
+enum SweepKernel {
+    SK_SWEEP = 0,   // k_sweep (mixed MHD with physical sides or refinement), k_sweep_hyd
+    SK_MX = 1,      // k_sweep_mx (mixed MHD, one level, periodic)
+    SK_64 = 2,      // k_sweep64 (FP64 MHD)
+    SK_64_NARROW = 3,   // ... where no wider tile fits the blocks
+    SK_64_TILE = 4      // ... when kr_config.tile asks for it: never the fastest
 };
+struct SweepVariant {
+    int tx, ty, nt, waves, kernel;
+};
+// k_sweep64: a 16x8 tile's solves of a plane fill 256 threads twice or 512
+// once.  Two workgroups of 256 overlap on a compute unit and win where the
+// tiles fill the GPU (128^3 in 32^3 blocks: 0.52 against 0.60 ms a launch);
+// one of 512 takes half as long over a plane where they do not (64^3: 93
+// against 112 us).  Likewise 8x8 with 320 threads (one round; 32^3 cells in
+// 16^3 blocks: 36 against 46 us) and 192 (two; 128^3: 0.94 against 1.17 ms).
 constexpr SweepVariant kSweepVariants[] = {
-    {32, 8, 512, 1, 0}, {32, 8, 512, 4, 0}, {16, 16, 512, 1, 0}, {16, 16, 512, 4, 0},
-    {16, 8, 256, 1, 0}, {8, 8, 192, 1, 0},  {16, 8, 256, 4, 0},  {16, 8, 256, 1, 1},
-    {32, 8, 512, 1, 1}, {16, 16, 512, 1, 1}, {8, 8, 192, 1, 1},
+    {32, 8, 512, 1, SK_SWEEP},  {32, 8, 512, 4, SK_SWEEP}, {16, 16, 512, 1, SK_SWEEP},
+    {16, 16, 512, 4, SK_SWEEP}, {16, 8, 256, 1, SK_SWEEP}, {8, 8, 192, 1, SK_SWEEP},
+    {16, 8, 256, 4, SK_SWEEP},  {16, 8, 256, 1, SK_MX},    {32, 8, 512, 1, SK_MX},
+    {16, 16, 512, 1, SK_MX},    {8, 8, 192, 1, SK_MX},     {32, 8, 512, 1, SK_64},
+    {16, 8, 512, 1, SK_64},     {16, 8, 256, 1, SK_64},    {8, 8, 320, 1, SK_64},
+    {16, 16, 512, 1, SK_64_TILE}, {8, 8, 192, 1, SK_64_NARROW},
 };
 constexpr int kNumSweepVariants = sizeof(kSweepVariants) / sizeof(kSweepVariants[0]);
 
@@ -216,8 +231,8 @@ struct kr_ctx {
     int4 *d_items = nullptr;        // its items (block, tile, z0, z1) and their count
     int *d_nitems = nullptr;
     int ncu = 0;                    // compute units (0: not asked yet)
-    int per_cu[16] = {0};           // resident workgroups per compute unit by variant, 15 the
-                                    // producer forms (0: not asked yet)
+    int per_cu[kNumSweepVariants + 1] = {0};   // resident workgroups per compute unit by variant,
+                                    // the last the producer forms (0: not asked yet)
     std::vector<int> candidates;    // variants the autotuner times
     int tune_next = 0;              // next candidate to time
     bool tuned = false;
@@ -255,7 +270,7 @@ struct kr_ctx {
     hipGraphExec_t graph = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     kr_stats stats{};
-    float tune_ms[16] = {0};
+    float tune_ms[kNumSweepVariants] = {0};
     std::vector<double> stage;   // host staging for packing
 
     template <class FT> MeshView<FT> view() const {
@@ -265,6 +280,8 @@ struct kr_ctx {
         m.nv = nv;
         for (int s = 0; s < 6; ++s) m.bnd[s] = cfg.bnd[s];
         m.gamma = cfg.gamma;
+        m.cv = 1 / (cfg.gamma - 1);
+        m.ge = 1 / m.cv + 1;
         for (int k = 0; k < 5; ++k) m.fix_w[k] = cfg.fix_w[k];
         for (int k = 0; k < 3; ++k) m.fix_b[k] = cfg.fix_b[k];
         m.cfl = cfg.cfl;
@@ -662,8 +679,12 @@ void commit(kr_ctx *c) {
         c->candidates.clear();
         for (int v = 0; v < kNumSweepVariants; ++v) {
             const SweepVariant &sv = kSweepVariants[v];
-            if (sv.mx && !mxmesh) continue;
-            if (mxmesh && !sv.mx && !(tx && tw > 1)) continue;
+            const bool f64 = c->mhd && !c->mixed;
+            if ((sv.kernel == SK_MX) && !mxmesh) continue;
+            if (mxmesh && sv.kernel == SK_SWEEP && !(tx && tw > 1)) continue;
+            if (f64 != (sv.kernel >= SK_64)) continue;
+            if (sv.kernel == SK_64_TILE && !tx) continue;
+            if (sv.kernel == SK_64_NARROW && c->n[0] % 16 == 0) continue;
             if (tx && (sv.tx != tx || sv.ty != ty)) continue;
             if (tw && sv.waves != tw) continue;
             if (sv.waves > 1 && (!c->mixed || !c->mhd)) continue;
@@ -781,6 +802,7 @@ struct Launcher {
     kr_ctx *c;
     bool prof = false;   // events around every launch
     bool tune = false;   // events around the fused stage-kernel launches only
+    bool again = false;  // the stage's fused launch may run twice (substep 0 reads slot 0 only)
     std::vector<std::pair<int, std::pair<hipEvent_t, hipEvent_t>>> evs;
 
     template <class F> void run(int kind, F &&f, bool sweep_launch = false) {
@@ -788,6 +810,9 @@ struct Launcher {
             f();
             return;
         }
+        // a kernel's first launch also loads its code (3x the time of the next
+        // one on a small mesh): tuning times the next
+        if (tune && again) f();
         hipEvent_t a, b;
         KR_HIP(hipEventCreate(&a));
         KR_HIP(hipEventCreate(&b));
@@ -816,36 +841,39 @@ struct Launcher {
         const int per = resident(variant, reinterpret_cast<const void *>(fn), threads);
         return z_ranges((size_t)nt * nb, c->ncu, per, c->n[2], lat);
     }
-    template <class FT, int TX, int TY, int NT, int W, int PROD = 0>
-    void sweep_t(const MeshView<FT> &m, int step, unsigned nb) {
-        const unsigned nt = (unsigned)((c->n[0] / TX) * (c->n[1] / TY));
-        auto go = [&](auto fn) {
-            const unsigned kz = ranges(fn, PROD ? 15 : c->variant, NT, nt, nb,
-                                       std::is_same_v<FT, double> ? kLatMhd64 : kLatMhdMixed);
-            hipLaunchKernelGGL(fn, dim3(nt, nb, kz), dim3(NT), 0, c->stream, m, step);
-        };
-        if (c->npfill)                      // physical sides (one-level meshes only)
-            go(k_sweep<FT, TX, TY, NT, W, PROD, true>);
-        else
-            go(k_sweep<FT, TX, TY, NT, W, PROD, false>);
+    template <class K, class FT>
+    void launch(K fn, const MeshView<FT> &m, int step, int variant, int tx, int ty, int threads,
+                unsigned nb, double lat) {
+        const unsigned nt = (unsigned)((c->n[0] / tx) * (c->n[1] / ty));
+        const unsigned kz = ranges(fn, variant, threads, nt, nb, lat);
+        hipLaunchKernelGGL(fn, dim3(nt, nb, kz), dim3(threads), 0, c->stream, m, step);
     }
-    // fluxes and edge EMFs of the listed blocks into F / EE (no update)
-    template <class FT> void sweep_prod(const MeshView<FT> &m, int step, unsigned nb) {
-        if (c->prod == 0) sweep_t<FT, 16, 8, 256, 1, 1>(m, step, nb);
-        else sweep_t<FT, 8, 8, 192, 1, 1>(m, step, nb);
+    template <int TX, int TY, int NT, int W, int PROD = 0>
+    void sweep_t(const MeshView<float> &m, int step, unsigned nb) {
+        // npfill: physical sides (one-level meshes only)
+        launch(c->npfill ? k_sweep<TX, TY, NT, W, PROD, true> : k_sweep<TX, TY, NT, W, PROD, false>, m,
+               step, PROD ? kNumSweepVariants : c->variant, TX, TY, NT, nb, kLatMhdMixed);
     }
-    template <class FT> void sweep_both(const MeshView<FT> &m, int step, unsigned nb) {
-        static_assert(std::is_same_v<FT, float>, "the combined launch is the mixed form's");
-        if (c->prod == 0) sweep_t<FT, 16, 8, 256, 1, 2>(m, step, nb);
-        else sweep_t<FT, 8, 8, 192, 1, 2>(m, step, nb);
+    template <int TX, int TY, int NT, int PROD = 0>
+    void sweep64_t(const MeshView<double> &m, int step, unsigned nb) {
+        launch(c->npfill ? k_sweep64<TX, TY, NT, PROD, true> : k_sweep64<TX, TY, NT, PROD, false>, m, step,
+               PROD ? kNumSweepVariants : c->variant, TX, TY, NT, nb, kLatMhd64);
+    }
+    // FP64: fluxes and edge EMFs of the listed blocks into F / EE (no update)
+    void sweep_prod(const MeshView<double> &m, int step, unsigned nb) {
+        if (c->prod == 0) sweep64_t<16, 8, 256, 1>(m, step, nb);
+        else if (nb * (unsigned)((c->n[0] / 8) * (c->n[1] / 8)) <= 512) sweep64_t<8, 8, 320, 1>(m, step, nb);
+        else sweep64_t<8, 8, 192, 1>(m, step, nb);
+    }
+    // mixed: the full form on the first rows, the producer form on the others
+    void sweep_both(const MeshView<float> &m, int step, unsigned nb) {
+        if (c->prod == 0) sweep_t<16, 8, 256, 1, 2>(m, step, nb);
+        else sweep_t<8, 8, 192, 1, 2>(m, step, nb);
     }
 
     template <class FT, int TX, int TY, int NT>
     void sweep_hyd_t(const MeshView<FT> &m, int step, unsigned nb) {
-        const unsigned nt = (unsigned)((c->n[0] / TX) * (c->n[1] / TY));
-        const auto fn = k_sweep_hyd<FT, TX, TY, NT>;
-        const unsigned kz = ranges(fn, c->variant, NT, nt, nb, kLatHydro);
-        hipLaunchKernelGGL(fn, dim3(nt, nb, kz), dim3(NT), 0, c->stream, m, step);
+        launch(k_sweep_hyd<FT, TX, TY, NT>, m, step, c->variant, TX, TY, NT, nb, kLatHydro);
     }
     // hydro: the one-wave-per-SIMD-minimum variants of the tile table
     template <class FT> void sweep_hyd(const MeshView<FT> &m, int step, int variant, unsigned nb) {
@@ -858,26 +886,29 @@ struct Launcher {
     }
 
     // grid rows: nb blocks (m.blist maps a row to its block when set)
-    template <class FT> void sweep(const MeshView<FT> &m, int step, int variant, unsigned nb) {
-        constexpr bool f32 = std::is_same_v<FT, float>;
+    void sweep(const MeshView<float> &m, int step, int variant, unsigned nb) {
         switch (variant) {
-        case 0: sweep_t<FT, 32, 8, 512, 1>(m, step, nb); break;
-        case 1: sweep_t<FT, 32, 8, 512, f32 ? 4 : 1>(m, step, nb); break;
-        case 2: sweep_t<FT, 16, 16, 512, 1>(m, step, nb); break;
-        case 3: sweep_t<FT, 16, 16, 512, f32 ? 4 : 1>(m, step, nb); break;
-        case 4: sweep_t<FT, 16, 8, 256, 1>(m, step, nb); break;
-        case 5: sweep_t<FT, 8, 8, 192, 1>(m, step, nb); break;
-        case 6: sweep_t<FT, 16, 8, 256, f32 ? 4 : 1>(m, step, nb); break;
-        default:
-            if constexpr (f32) {
-                switch (variant) {
-                case 7: sweep_mx_t<16, 8, 256>(m, step, nb); break;
-                case 8: sweep_mx_t<32, 8, 512>(m, step, nb); break;
-                case 9: sweep_mx_t<16, 16, 512>(m, step, nb); break;
-                default: sweep_mx_t<8, 8, 192>(m, step, nb); break;
-                }
-            }
-            break;
+        case 0: sweep_t<32, 8, 512, 1>(m, step, nb); break;
+        case 1: sweep_t<32, 8, 512, 4>(m, step, nb); break;
+        case 2: sweep_t<16, 16, 512, 1>(m, step, nb); break;
+        case 3: sweep_t<16, 16, 512, 4>(m, step, nb); break;
+        case 4: sweep_t<16, 8, 256, 1>(m, step, nb); break;
+        case 5: sweep_t<8, 8, 192, 1>(m, step, nb); break;
+        case 6: sweep_t<16, 8, 256, 4>(m, step, nb); break;
+        case 7: sweep_mx_t<16, 8, 256>(m, step, nb); break;
+        case 8: sweep_mx_t<32, 8, 512>(m, step, nb); break;
+        case 9: sweep_mx_t<16, 16, 512>(m, step, nb); break;
+        default: sweep_mx_t<8, 8, 192>(m, step, nb); break;
+        }
+    }
+    void sweep(const MeshView<double> &m, int step, int variant, unsigned nb) {
+        switch (variant) {
+        case 11: sweep64_t<32, 8, 512>(m, step, nb); break;
+        case 12: sweep64_t<16, 8, 512>(m, step, nb); break;
+        case 13: sweep64_t<16, 8, 256>(m, step, nb); break;
+        case 14: sweep64_t<8, 8, 320>(m, step, nb); break;
+        case 15: sweep64_t<16, 16, 512>(m, step, nb); break;
+        default: sweep64_t<8, 8, 192>(m, step, nb); break;
         }
     }
     // Ensembles: the stage's work list (the tiles of the boxes still
@@ -906,6 +937,7 @@ struct Launcher {
     }
 
     template <class FT, bool MHD> void stage(int step) {
+        again = step == 0;
         const MeshView<FT> m = c->view<FT>();
         const unsigned nb = (unsigned)c->descs.size();
         const dim3 blk(kThreads);
@@ -929,7 +961,7 @@ struct Launcher {
                                        dim3(256), 0, c->stream, m, (const int4 *)c->d_pfill);
                 });
             if constexpr (MHD)
-                run(KR_K_UPDATE, [&] { sweep<FT>(m, step, c->variant, nb); }, true);
+                run(KR_K_UPDATE, [&] { sweep(m, step, c->variant, nb); }, true);
             else
                 run(KR_K_UPDATE, [&] { sweep_hyd<FT>(m, step, c->variant, nb); }, true);
             return;
@@ -964,14 +996,14 @@ struct Launcher {
                     mb.blist = c->d_sweep;
                     mb.nfull = c->npure;
                     run(KR_K_UPDATE,
-                        [&] { sweep_both<FT>(mb, step, (unsigned)(c->npure + c->nxblk)); }, true);
+                        [&] { sweep_both(mb, step, (unsigned)(c->npure + c->nxblk)); }, true);
                     both = true;
                 }
             if (!both && c->npure) {
                 MeshView<FT> mp = m;
                 mp.blist = c->d_pure;
                 if constexpr (MHD)
-                    run(KR_K_UPDATE, [&] { sweep<FT>(mp, step, c->variant, (unsigned)c->npure); }, true);
+                    run(KR_K_UPDATE, [&] { sweep(mp, step, c->variant, (unsigned)c->npure); }, true);
                 else
                     run(KR_K_UPDATE, [&] { sweep_hyd<FT>(mp, step, c->variant, (unsigned)c->npure); },
                         true);
@@ -984,7 +1016,7 @@ struct Launcher {
             // producer form: fluxes and EMFs into F / EE (the mixed form ran
             // it in the launch above)
             if constexpr (!std::is_same_v<FT, float>)
-                run(KR_K_FLUX_X, [&] { sweep_prod<FT>(ms, step, ns); });
+                run(KR_K_FLUX_X, [&] { sweep_prod(ms, step, ns); });
         } else {
         if (c->ndim > 2)
             run(KR_K_FLUX_Z, [&] {
@@ -1074,7 +1106,7 @@ void fill_tile_stats(kr_ctx *c) {
     c->stats.sweep_tile[1] = sv.ty;
     c->stats.sweep_tile[2] = sv.nt;
     c->stats.sweep_tile[3] = sv.waves;
-    c->stats.sweep_kernel = sv.mx;
+    c->stats.sweep_kernel = sv.kernel == SK_MX;
     for (int v = 0; v < kNumSweepVariants && v < 16; ++v) c->stats.tune_ms[v] = c->tune_ms[v];
 }
 

@@ -12,11 +12,12 @@
 //   4. update: Heun slot of the cells of plane L-2 (x, y parts were
 //      accumulated one iteration earlier, z part now) and CT of the faces of
 //      plane L-2 and z-face L-1.
-// Arithmetic is the same per-face restatement as the staged kernels
-// (kr_physics.h), in the same order, so both paths agree bit for bit in the
-// FP64 form.  PLM is evaluated per cell: the reference's two face states of
-// a cell share one limited increment t, q_l(face i+1) = q_i + t and
-// q_r(face i) = q_i + (-t) exactly (hydro/reconstruct/plm.h:116-153).
+// k_sweep is the mixed form's kernel (FP32 fluxes, FP64 state) for meshes
+// with physical sides and refined ones; kr_sweep_mx.h has the one for
+// one-level periodic meshes, kr_sweep64.h the FP64 form's.  PLM is evaluated
+// per cell: the reference's two face states of a cell share one limited
+// increment t, q_l(face i+1) = q_i + t and q_r(face i) = q_i + (-t) exactly
+// (hydro/reconstruct/plm.h:116-153).
 #pragma once
 
 #include "kr_staged.h"
@@ -71,27 +72,6 @@ __device__ __forceinline__ void z_range(int nz, int &z0, int &z1) {
 
 __device__ __forceinline__ int ring3(int p) { return ((p % 3) + 3) % 3; }
 __device__ __forceinline__ int ring2(int p) { return (p + 4) & 1; }
-
-// Per-cell PLM increment of one variable (see header): returns t with the
-// reference's expression order; `flat` is the reference's dq2 <= 0 branch.
-template <class FT>
-__device__ __forceinline__ FT plm_inc(FT qm, FT q0, FT qp, bool &flat) {
-    const FT dql = q0 - qm;
-    const FT dqc = qp - q0;
-    FT norm(1);
-    if constexpr (std::is_same_v<FT, float>) {
-        // FP32: the slope ratio is scale free; rescale by the larger
-        // difference so the squares stay in range (plm.h:128-137 in spirit)
-        const FT s = pmax(kfabs(dql), kfabs(dqc));
-        if (s > (FT)1e-24f) norm = 1 / s;
-    }
-    const FT dql2 = norm * dql * dql;
-    const FT dqc2 = norm * dqc * dqc;
-    const FT dq2 = norm * dql * dqc;
-    flat = dq2 <= 0;
-    const FT coef = flat ? (FT)0 : dq2 / (dql2 + dqc2 + dq2 * 2);
-    return coef * (dql + dqc);
-}
 
 // a * b - c * d in FP32 with multiply-add contraction (mixed form)
 __device__ __forceinline__ float cross_f32(float a, float b, float c, float d) {
@@ -174,9 +154,10 @@ __device__ __forceinline__ double edge_emf<double>(double ec11, double ec10, dou
 // PROD = 2 (refined meshes): one launch for both kinds of block, the grid
 // rows below m.nfull updating (the full form), the rows from m.nfull on
 // producing (the producer form); a workgroup takes its row's form.
-template <class FT, int TX, int TY, int NT, int WAVES, int PROD = 0, bool PHY = false>
+template <int TX, int TY, int NT, int WAVES, int PROD = 0, bool PHY = false>
 __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WAVES)))
-k_sweep(MeshView<FT> m, int step) {
+k_sweep(MeshView<float> m, int step) {
+    using FT = float;
     using S = TileShape<TX, TY>;
     static_assert(S::NCOL <= NT, "one halo column per thread");
     static_assert(S::NZIP <= NT, "one z pencil per thread, in-plane items from a wave boundary");
@@ -222,8 +203,7 @@ k_sweep(MeshView<FT> m, int step) {
     // Per-block factors of the update and the CT, formed once per launch
     // (the same expressions as at each use, so the same values): CT factor
     // -dt / sfc_a, flux factor sfc_a * dt / vol, edge length dx_a.  Kept in
-    // LDS, not registers, and read where used by the FP32 flux form; the
-    // FP64 form forms them at each use (its code is faster that way).
+    // LDS, not registers, and read where used.
     __shared__ double sGeo[9];
     if (tid < 3) {
         const double sfc = g.sfc[tid];
@@ -354,10 +334,6 @@ k_sweep(MeshView<FT> m, int step) {
     const bool xedge = xlast && et >= 0 && et < TY;
     const bool yedge = ylast && et >= TY && et < TY + TX;
 
-    constexpr bool F32 = std::is_same_v<FT, float>;
-    const double dt_dv = dt / g.vol;
-
-
     issue_w(z0 - 2, ring3(z0 - 2));
     for (int L = z0 - 2; L <= z1 + 1; ++L) {
         // ------------------------------------------------ 1. plane L arrives
@@ -384,16 +360,9 @@ k_sweep(MeshView<FT> m, int step) {
                         continue;
                     }
                     const FT q0 = sW[s0][v][c];
-                    if constexpr (std::is_same_v<FT, float>) {
-                        const float t = plm_inc_fast(sW[sm][v][c], q0, sW[sp][v][c]);
-                        qR[v] = q0 - t;
-                        qLn[v] = q0 + t;
-                    } else {
-                        bool flat;
-                        const FT t = plm_inc<FT>(sW[sm][v][c], q0, sW[sp][v][c], flat);
-                        qR[v] = q0 + (flat ? (FT)0 : -t);
-                        qLn[v] = q0 + (flat ? (FT)0 : t);
-                    }
+                    const float t = plm_inc_fast(sW[sm][v][c], q0, sW[sp][v][c]);
+                    qR[v] = q0 - t;
+                    qLn[v] = q0 + t;
                 }
                 if (p >= z0) {
                     FT wl[8], wr[8], flx[8];
@@ -409,10 +378,7 @@ k_sweep(MeshView<FT> m, int step) {
                     rot<2>(wr + MOM);
                     rot<2>(wl + BCC);
                     rot<2>(wr + BCC);
-                    if constexpr (std::is_same_v<FT, float>)
-                        hlld_fast(flx, wl, wr, gam);
-                    else
-                        hlld<FT>(flx, wl, wr, gam);
+                    hlld_fast(flx, wl, wr, gam);
                     rot<1>(flx + MOM);
                     // EMF rewrite for axis 2: E_x = flx[BCC+2], E_y = -flx[BCC+1]
                     const int gz = S::zg(zx, zy);
@@ -428,19 +394,14 @@ k_sweep(MeshView<FT> m, int step) {
                     } else if (!prod && zint) {
                         // z part of the cell finished now (plane p-1 = P)
                         if (P >= z0) {
-                            const FT fa = F32 ? (FT)sGeo[3 + 2] : (FT)(g.sfc[2] * dt_dv);
+                            const FT fa = (FT)sGeo[3 + 2];
                             const size_t cc = cidx(m.n, x0 + cx_, y0 + cy_, P);
                             double *Ut = m.U + ((size_t)b * 2 + (1 - step)) * 5 * nc + cc;
 #pragma unroll
                             for (int v = 0; v < 5; ++v) {
                                 double res(0);
-                                if constexpr (std::is_same_v<FT, double>) {
-                                    if (fa > 0) res += fa * fzp[v];
-                                    if (fa > 0) res -= fa * flx[v];
-                                } else {
-                                    if (fa > 0) res += (double)(fa * fzp[v]);
-                                    if (fa > 0) res -= (double)(fa * flx[v]);
-                                }
+                                if (fa > 0) res += (double)(fa * fzp[v]);
+                                if (fa > 0) res -= (double)(fa * flx[v]);
                                 Ut[(size_t)v * nc] = part[v] + res;
                             }
                         }
@@ -483,23 +444,12 @@ k_sweep(MeshView<FT> m, int step) {
                     const FT *q = &sW[s0][v][0];
                     const FT qm2 = q[cR - 2 * stride], qm1 = q[cR - stride];
                     const FT q00 = q[cR], qp1 = q[cR + stride];
-                    if constexpr (std::is_same_v<FT, float>) {
-                        plm_fast(qm2, qm1, q00, qp1, wl[k], wr[k]);
-                    } else {
-                        bool fl, fr;
-                        const FT tl = plm_inc<FT>(qm2, qm1, q00, fl);
-                        const FT tr = plm_inc<FT>(qm1, q00, qp1, fr);
-                        wl[k] = qm1 + (fl ? (FT)0 : tl);
-                        wr[k] = q00 + (fr ? (FT)0 : -tr);
-                    }
+                    plm_fast(qm2, qm1, q00, qp1, wl[k], wr[k]);
                 }
                 const FT bn = bfn(a, fx, fy, p, s0);
                 wl[BCC] = bn;
                 wr[BCC] = bn;
-                if constexpr (std::is_same_v<FT, float>)
-                    hlld_fast(flx, wl, wr, gam);
-                else
-                    hlld<FT>(flx, wl, wr, gam);
+                hlld_fast(flx, wl, wr, gam);
                 // back to the mesh frame
                 sFh[0][it] = flx[ENE];
 #pragma unroll
@@ -541,10 +491,7 @@ k_sweep(MeshView<FT> m, int step) {
                 const int c1 = (c + 1) % 3, c2 = (c + 2) % 3;
                 const FT b1 = sW[s][BCC + c1][cc], v2 = sW[s][MOM + c2][cc];
                 const FT b2 = sW[s][BCC + c2][cc], v1 = sW[s][MOM + c1][cc];
-                if constexpr (std::is_same_v<FT, float>)
-                    return cross_f32(b1, v2, b2, v1);
-                else
-                    return b1 * v2 - b2 * v1;
+                return cross_f32(b1, v2, b2, v1);
             };
             // boundary-plane EMF of a high out / fre side
             // (mhd/integrator/integrator.h:328-381), as k_emf: edge c at
@@ -662,16 +609,10 @@ k_sweep(MeshView<FT> m, int step) {
                 db -= e2 * d2;
                 db += e3 * d2;
                 db -= e4 * d1;
-                if constexpr (F32) {
-                    db *= sGeo[a];              // -dt / sfc, or 0 for a zero-area face
-                } else {
-                    const double sfc = g.sfc[a];
-                    db *= (sfc > 0 ? (double)(-dt / sfc) : (double)(0));
-                }
+                db *= sGeo[a];              // -dt / sfc, or 0 for a zero-area face
                 return db;
             };
-            const double dx = F32 ? sGeo[6] : g.dx[0], dy = F32 ? sGeo[7] : g.dx[1],
-                         dz = F32 ? sGeo[8] : g.dx[2];
+            const double dx = sGeo[6], dy = sGeo[7], dz = sGeo[8];
             if (zint) {
                 const int x = cx_, y = cy_;
                 const FaceUpd uz = face_load(2, x, y, q);
@@ -696,28 +637,15 @@ k_sweep(MeshView<FT> m, int step) {
                     for (int a = 0; a < 2; ++a) {
                         const int i0 = a == 0 ? S::fxi(x, y) : S::fyi(x, y);
                         const int i1 = a == 0 ? S::fxi(x + 1, y) : S::fyi(x, y + 1);
-                        if constexpr (std::is_same_v<FT, double>) {
-                            const double fa = g.sfc[a] * dt_dv;
+                        const float fa = (float)sGeo[3 + a];
 #pragma unroll
-                            for (int v = 0; v < 5; ++v) {
-                                double res(0);
-                                const FT f0 = v == 0 ? sFe[fq][0][i0] : sFh[v - 1][i0];
-                                const FT f1 = v == 0 ? sFe[fq][0][i1] : sFh[v - 1][i1];
-                                if (fa > 0) res += fa * f0;
-                                if (fa > 0) res -= fa * f1;
-                                uu[v] += res;
-                            }
-                        } else {
-                            const float fa = (float)sGeo[3 + a];
-#pragma unroll
-                            for (int v = 0; v < 5; ++v) {
-                                double res(0);
-                                const FT f0 = v == 0 ? sFe[fq][0][i0] : sFh[v - 1][i0];
-                                const FT f1 = v == 0 ? sFe[fq][0][i1] : sFh[v - 1][i1];
-                                if (fa > 0) res += (double)(fa * f0);
-                                if (fa > 0) res -= (double)(fa * f1);
-                                uu[v] += res;
-                            }
+                        for (int v = 0; v < 5; ++v) {
+                            double res(0);
+                            const FT f0 = v == 0 ? sFe[fq][0][i0] : sFh[v - 1][i0];
+                            const FT f1 = v == 0 ? sFe[fq][0][i1] : sFh[v - 1][i1];
+                            if (fa > 0) res += (double)(fa * f0);
+                            if (fa > 0) res -= (double)(fa * f1);
+                            uu[v] += res;
                         }
                     }
 #pragma unroll

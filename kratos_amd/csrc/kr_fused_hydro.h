@@ -24,6 +24,7 @@
 // hllc.h:32-193; rk2.h:20-41.
 #pragma once
 
+#include "kr_exact64.h"
 #include "kr_fused.h"
 
 namespace kr {
@@ -46,6 +47,7 @@ __global__ void __launch_bounds__(NT) k_sweep_hyd(MeshView<FT> m, int step) {
     const BlockGeo &g = m.geo[b];
     const double dt = m.ts[g.grp].dt_use * (step == 0 ? 1.0 : 0.5);
     const FT gam = (FT)m.gamma;
+    const Gam64 gam64{m.gamma, m.cv, m.ge};
     const size_t nc = m.ncell;
 
     constexpr int DPC = (int)sizeof(FT) / 4;                   // dwords per column
@@ -131,19 +133,25 @@ __global__ void __launch_bounds__(NT) k_sweep_hyd(MeshView<FT> m, int step) {
             if (own) {
                 const int c = S::col(cx, cy);
                 FT qR[5], qLn[5];
+                FT t[5];
+                if constexpr (F32) {
+#pragma unroll
+                    for (int v = 0; v < 5; ++v)
+                        t[v] = plm_inc_fast(sW[sm][v][c], sW[s0][v][c], sW[sp][v][c]);
+                } else {
+                    FT lo[5], hi[5];
+#pragma unroll
+                    for (int v = 0; v < 5; ++v) {
+                        lo[v] = sW[s0][v][c] - sW[sm][v][c];
+                        hi[v] = sW[sp][v][c] - sW[s0][v][c];
+                    }
+                    plm_inc64<5>(lo, hi, t);
+                }
 #pragma unroll
                 for (int v = 0; v < 5; ++v) {
                     const FT q0 = sW[s0][v][c];
-                    if constexpr (std::is_same_v<FT, float>) {
-                        const float t = plm_inc_fast(sW[sm][v][c], q0, sW[sp][v][c]);
-                        qR[v] = q0 - t;
-                        qLn[v] = q0 + t;
-                    } else {
-                        bool flat;
-                        const FT t = plm_inc<FT>(sW[sm][v][c], q0, sW[sp][v][c], flat);
-                        qR[v] = q0 + (flat ? (FT)0 : -t);
-                        qLn[v] = q0 + (flat ? (FT)0 : t);
-                    }
+                    qR[v] = q0 - t[v];
+                    qLn[v] = q0 + t[v];
                 }
                 if (p >= z0) {
                     FT wl[5], wr[5], flx[5];
@@ -157,7 +165,7 @@ __global__ void __launch_bounds__(NT) k_sweep_hyd(MeshView<FT> m, int step) {
                     if constexpr (std::is_same_v<FT, float>)
                         hllc_fast(flx, wl, wr, gam);
                     else
-                        hllc<FT>(flx, wl, wr, gam);
+                        hllc64(flx, wl, wr, gam64);
                     rot<1>(flx + MOM);
                     if (P >= z0) {
                         // z part of cell P: faces P (previous) and p = P + 1
@@ -201,7 +209,7 @@ __global__ void __launch_bounds__(NT) k_sweep_hyd(MeshView<FT> m, int step) {
                     const int a = xf ? 0 : 1;
                     const int stride = xf ? 1 : S::HX;
                     const int cR = S::col(fx, fy);      // cell on the right of the face
-                    FT wl[5], wr[5], flx[5];
+                    FT wl[5], wr[5], flx[5], lo[10], hi[10], t[10];
                     // rotated frame: slot k holds mesh variable perm(k)
 #pragma unroll
                     for (int k = 0; k < 5; ++k) {
@@ -210,20 +218,28 @@ __global__ void __launch_bounds__(NT) k_sweep_hyd(MeshView<FT> m, int step) {
                         const FT *q = &sW[s0][v][0];
                         const FT qm2 = q[cR - 2 * stride], qm1 = q[cR - stride];
                         const FT q00 = q[cR], qp1 = q[cR + stride];
-                        if constexpr (std::is_same_v<FT, float>) {
+                        if constexpr (F32) {
                             plm_fast(qm2, qm1, q00, qp1, wl[k], wr[k]);
                         } else {
-                            bool fl, fr;
-                            const FT tl = plm_inc<FT>(qm2, qm1, q00, fl);
-                            const FT tr = plm_inc<FT>(qm1, q00, qp1, fr);
-                            wl[k] = qm1 + (fl ? (FT)0 : tl);
-                            wr[k] = q00 + (fr ? (FT)0 : -tr);
+                            wl[k] = qm1;
+                            wr[k] = q00;
+                            lo[k] = qm1 - qm2;
+                            hi[k] = lo[5 + k] = q00 - qm1;
+                            hi[5 + k] = qp1 - q00;
+                        }
+                    }
+                    if constexpr (!F32) {
+                        plm_inc64<10>(lo, hi, t);
+#pragma unroll
+                        for (int k = 0; k < 5; ++k) {
+                            wl[k] += t[k];
+                            wr[k] -= t[5 + k];
                         }
                     }
                     if constexpr (std::is_same_v<FT, float>)
                         hllc_fast(flx, wl, wr, gam);
                     else
-                        hllc<FT>(flx, wl, wr, gam);
+                        hllc64(flx, wl, wr, gam64);
                     sF[RHO][it] = flx[RHO];
                     sF[ENE][it] = flx[ENE];
 #pragma unroll

@@ -84,6 +84,7 @@ struct MeshView {
     int nv;            // variables in W and F: 5 hydro, 8 MHD
     int bnd[6];        // boundary kind per side (0 per, 1 out, 2 fre, 3 ref, 4 fixd)
     double gamma, cfl, d_floor, t_floor;
+    double cv, ge;     // 1 / (gamma - 1) and 1 / cv + 1 (the FP64 flux functions)
     double fix_w[5], fix_b[3];   // fixd ghost primitives and B
     size_t ncell;      // n0*n1*n2
     size_t nface;      // (n0+1)(n1+1)(n2+1): face / edge box
