@@ -4,6 +4,7 @@
 #include "../../include/kratos_amd.h"
 #include "kr_fused.h"
 #include "kr_fused_hydro.h"
+#include "kr_plane.h"
 #include "kr_smr.h"
 #include "kr_sweep64.h"
 #include "kr_sweep_mx.h"
@@ -35,11 +36,9 @@ __global__ void k_cycle_begin(TimeState *tsv, int ngrp) {
     if (!ts->skip) ts->cycles += 1;
 }
 
-// Global CFL reduction and the dt / t bookkeeping of redc_dt_start/finish
-// (mesh/cycle/cycle.cpp:77-115): p_dt = min(p_dt, CFL), dt_use clamped to
-// t_lim when topping up, t advanced, next seed = dt_use * dt_expand.  One
-// workgroup per time group; the group's blocks are contiguous, so its CFL
-// partials are part[grp_first[g] * ppb, grp_first[g + 1] * ppb).
+// dt of every time group from its CFL partials (take_dt).  One workgroup per
+// time group; the group's blocks are contiguous, so its CFL partials are
+// part[grp_first[g] * ppb, grp_first[g + 1] * ppb).
 __global__ void __launch_bounds__(1024) k_dt_finalize(TimeState *tsv, const double *part,
                                                       const int *grp_first, int ppb) {
     TimeState *ts = tsv + blockIdx.x;
@@ -55,16 +54,7 @@ __global__ void __launch_bounds__(1024) k_dt_finalize(TimeState *tsv, const doub
     __syncthreads();
     if (threadIdx.x == 0) {
         for (int i = 1; i < (int)(blockDim.x >> 6); ++i) v = pmin(v, red[i]);
-        const double p = __builtin_fmin(v, ts->p_dt);
-        const double dt_use = ts->top_up ? (p < ts->t_lim - ts->t ? p : ts->t_lim - ts->t) : p;
-        if (ts->top_up) {
-            const double tn = dt_use + ts->t;
-            ts->t = tn < ts->t_lim ? tn : ts->t_lim;
-        } else {
-            ts->t = dt_use + ts->t;
-        }
-        ts->dt_use = dt_use;
-        ts->p_dt = dt_use * ts->dt_expand;
+        take_dt(ts, v);
     }
 }
 
@@ -171,6 +161,11 @@ unsigned z_ranges(size_t wgs, int ncu, int per_cu, int nz, double lat) {
     return best;
 }
 
+// Most c2p workgroups of a mesh whose last one takes the dt (FIN): up to
+// there the arrivals cost less than the two launches they replace (32^3: 128
+// workgroups, 92 -> 85 us a cycle).
+constexpr size_t kFinWorkgroups = 1024;
+
 // graph replays between host checks of the stop rule in kr_advance
 constexpr int kAdvanceChunk = 64;
 
@@ -225,6 +220,9 @@ struct kr_ctx {
     bool committed = false;
     bool mhd = false, mixed = false;
     bool fused = false;
+    bool plane = false;             // 1-D / 2-D mesh: a stage is one launch of k_plane
+    bool fin = false;               // k_c2p takes the dt itself (FIN)
+    int *arrived = nullptr;         // [ngrp] its workgroups done so far
     int variant = -1;               // kSweepVariants index of the fused kernel
     int prod = -1;                  // refined mesh: producer tile (0: 16x8, 1: 8x8), -1 none
     bool mx_list = false;           // k_sweep_mx walks a device work list (ensembles)
@@ -311,7 +309,7 @@ void release(kr_ctx *c) {
     void *bufs[] = {c->U,  c->BF, c->W,       c->F[0],  c->F[1],   c->F[2],  c->EE, c->EC,
                     c->geo, c->ts, c->grp_first, c->dt_part, c->red_part, c->red_out,
                     c->d_table, c->d_fill[0], c->d_fill[1], c->d_ftask, c->d_xblk,
-                    c->d_pure, c->d_pfill, c->d_sweep, c->d_items, c->d_nitems};
+                    c->d_pure, c->d_pfill, c->d_sweep, c->d_items, c->d_nitems, c->arrived};
     for (void *p : bufs)
         if (p) (void)hipFree(p);
     c->d_table = nullptr;
@@ -321,6 +319,7 @@ void release(kr_ctx *c) {
     c->d_xblk = c->d_pure = c->d_sweep = nullptr;
     c->d_items = nullptr;
     c->d_nitems = nullptr;
+    c->arrived = nullptr;
     c->U = c->BF = nullptr;
     c->W = c->EE = c->EC = nullptr;
     c->F[0] = c->F[1] = c->F[2] = nullptr;
@@ -738,8 +737,10 @@ void commit(kr_ctx *c) {
     c->U = dalloc<double>(nb * 2 * 5 * c->ncell);
     if (c->mhd) c->BF = dalloc<double>(nb * 2 * 3 * c->nface);
     KR_HIP(hipMalloc(&c->W, nw * c->nv * c->ncell * fs));
-    for (int a = 0; a < c->ndim; ++a) KR_HIP(hipMalloc(&c->F[a], nb * c->nv * c->nfa[a] * fs));
-    if (c->mhd) KR_HIP(hipMalloc(&c->EE, nb * 3 * c->nface * fs));
+    c->plane = c->ndim < 3 && c->cfg.kernel_path == KR_PATH_AUTO;
+    for (int a = 0; a < c->ndim && !c->plane; ++a)
+        KR_HIP(hipMalloc(&c->F[a], nb * c->nv * c->nfa[a] * fs));
+    if (c->mhd && !c->plane) KR_HIP(hipMalloc(&c->EE, nb * 3 * c->nface * fs));
     KR_HIP(hipMemset(c->U, 0, nb * 2 * 5 * c->ncell * sizeof(double)));
     if (c->mhd) KR_HIP(hipMemset(c->BF, 0, nb * 2 * 3 * c->nface * sizeof(double)));
     KR_HIP(hipMemset(c->W, 0, nw * c->nv * c->ncell * fs));
@@ -765,6 +766,9 @@ void commit(kr_ctx *c) {
 
     c->ppb = (int)ceil_div(c->ncell, kThreads);
     c->n_dt_part = nb * c->ppb;
+    c->fin = c->n_dt_part <= kFinWorkgroups;
+    c->arrived = dalloc<int>(c->ngrp);
+    KR_HIP(hipMemset(c->arrived, 0, c->ngrp * sizeof(int)));
     c->dt_part = dalloc<double>(c->n_dt_part);
     c->n_red_part = c->n_dt_part;
     c->red_part = dalloc<double>(c->n_red_part);
@@ -788,7 +792,7 @@ void commit(kr_ctx *c) {
         c->tune_next = 0;
     }
     // cell-centred E for the staged EMF kernel, when it runs
-    if (c->mhd && (!c->fused || (c->smr && c->prod < 0)))
+    if (c->mhd && !c->plane && (!c->fused || (c->smr && c->prod < 0)))
         KR_HIP(hipMalloc(&c->EC, nb * 3 * c->ncell * fs));
     c->stats.n_blocks = (int)nb;
     c->stats.n_cells = (long long)(nb * c->ncell);
@@ -936,21 +940,42 @@ struct Launcher {
                            step, (const int4 *)c->d_items, (const int *)c->d_nitems);
     }
 
+    // 2-D: an 8x8 tile's faces (180 for MHD) are one round of three waves,
+    // and its 12x12 halo one cell a thread; 1-D: 124 cells and 4 of halo
+    template <class FT, bool MHD, bool C2P> void plane(const MeshView<FT> &m, int step, unsigned nb) {
+        if (c->ndim > 1)
+            hipLaunchKernelGGL((k_plane<FT, MHD, 8, 8, 192, C2P>),
+                               dim3(ceil_div(c->n[0], 8) * ceil_div(c->n[1], 8), nb), dim3(192), 0,
+                               c->stream, m, step);
+        else
+            hipLaunchKernelGGL((k_plane<FT, MHD, 124, 1, 128, C2P>), dim3(ceil_div(c->n[0], 124), nb),
+                               dim3(128), 0, c->stream, m, step);
+    }
+
     template <class FT, bool MHD> void stage(int step) {
         again = step == 0;
         const MeshView<FT> m = c->view<FT>();
         const unsigned nb = (unsigned)c->descs.size();
         const dim3 blk(kThreads);
+        if (c->plane && step == 1) {        // substep 1 forms its own primitives
+            run(KR_K_UPDATE, [&] { plane<FT, MHD, true>(m, step, nb); });
+            return;
+        }
         run(KR_K_C2P, [&] {
-            hipLaunchKernelGGL((k_c2p<FT, MHD>), dim3(ceil_div(c->ncell, kThreads), nb), blk, 0,
-                               c->stream, m, step);
+            const auto fn = c->fin && step == 0 ? k_c2p<FT, MHD, true> : k_c2p<FT, MHD, false>;
+            hipLaunchKernelGGL(fn, dim3(ceil_div(c->ncell, kThreads), nb), blk, 0, c->stream, m, step,
+                               (const int *)c->grp_first, c->arrived);
         });
-        if (step == 0)
+        if (step == 0 && !c->fin)
             run(KR_K_DTFIN, [&] {
                 hipLaunchKernelGGL(k_dt_finalize, dim3(c->ngrp), dim3(1024), 0, c->stream, c->ts,
                                    (const double *)c->dt_part, (const int *)c->grp_first,
                                    c->ppb);
             });
+        if (c->plane) {
+            run(KR_K_UPDATE, [&] { plane<FT, MHD, false>(m, step, nb); });
+            return;
+        }
         constexpr int NV = MHD ? 8 : 5;
         if (c->fused && !c->smr) {
             if (c->npfill)                  // physical-side halos (accounted as c2p)
@@ -1075,7 +1100,7 @@ struct Launcher {
     }
 
     template <class FT, bool MHD> void cycle_t() {
-        run(KR_K_BEGIN, [&] {
+        if (!c->fin) run(KR_K_BEGIN, [&] {
             hipLaunchKernelGGL(k_cycle_begin, dim3(ceil_div(c->ngrp, 256)), dim3(256), 0,
                                c->stream, c->ts, c->ngrp);
         });

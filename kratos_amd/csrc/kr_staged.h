@@ -41,13 +41,23 @@ __device__ __forceinline__ int nbr_dir(const MeshView<FT> &m, const int *d) {
     return ((d[2] + 1) * 3 + (d[1] + 1)) * 3 + (d[0] + 1);
 }
 
-// Load the primitive vector of cell p of block b.  Cells outside the block
-// come from the same-level neighbour (the reference fills them by the
-// ghost exchange, hydro/boundary/comm_functions.h:304-327); on a physical
-// side the reference's boundary functor is applied on the fly
+// Where the primitives of a cell come from: cell p of block blk, then the
+// boundary functor of a physical side.
+struct CellSrc {
+    int blk, p[3];
+    int flip;       // axis of a reflecting side, -1: none
+    int clamp;      // 2 * axis + side of an outflow side, -1: none
+    bool fixd;      // Dirichlet side: the ghost is the fixed state
+};
+
+// Source of cell pin of block b.  Cells outside the block come from the
+// same-level neighbour (the reference fills them by the ghost exchange,
+// hydro/boundary/comm_functions.h:304-327); on a physical side the
+// reference's boundary functor is applied on the fly
 // (hydro/boundary/phys_functors.h:10-89).
 template <class FT, int NV>
-__device__ __forceinline__ void load_cell(const MeshView<FT> &m, int b, const int *pin, FT *w) {
+__device__ __forceinline__ CellSrc cell_src(const MeshView<FT> &m, int b, const int *pin) {
+    CellSrc c;
     int p[3] = {pin[0], pin[1], pin[2]};
     int d[3];
     bool out = false;
@@ -56,15 +66,14 @@ __device__ __forceinline__ void load_cell(const MeshView<FT> &m, int b, const in
         d[a] = p[a] < 0 ? -1 : (p[a] >= m.n[a] ? 1 : 0);
         out |= d[a] != 0;
     }
-    int blk = b;
-    int flip = -1;      // reflect: negate v_ax;  outflow: clamp inflow of v_ax
-    int clamp = -1;     // 2*ax + side of an outflow side
-    bool phys8 = false; // MHD cell behind a physical side
-    bool fixd = false;  // Dirichlet side: the ghost is the fixed state
+    c.blk = b;
+    c.flip = -1;
+    c.clamp = -1;
+    c.fixd = false;
     if (out) {
         const int nb = m.geo[b].nbr[nbr_dir(m, d)];
         if (nb >= 0) {
-            blk = nb;
+            c.blk = nb;
 #pragma unroll
             for (int a = 0; a < 3; ++a) p[a] -= d[a] * m.n[a];
         } else if constexpr (NV == 5) {
@@ -79,22 +88,16 @@ __device__ __forceinline__ void load_cell(const MeshView<FT> &m, int b, const in
                 const int g = side ? p[a] - m.n[a] : -1 - p[a];
                 if (kind == 3) {                       // reflect
                     p[a] = side ? m.n[a] - 1 - g : g;
-                    flip = a;
+                    c.flip = a;
                 } else {                               // outflow / free / fixd
                     p[a] = side ? m.n[a] - 1 : 0;
-                    if (kind == 1) clamp = 2 * a + side;
-                    if (kind == 4) fixd = true;
+                    if (kind == 1) c.clamp = 2 * a + side;
+                    if (kind == 4) c.fixd = true;
                 }
             }
 #pragma unroll
             for (int a = 0; a < 3; ++a) p[a] = p[a] < 0 ? 0 : (p[a] >= m.n[a] ? m.n[a] - 1 : p[a]);
         } else {
-            phys8 = true;
-        }
-    }
-    int mflip = -1, mclamp = -1;       // MHD physical side: reflect axis / outflow side
-    if constexpr (NV == 8) {
-        if (phys8) {
             // MHD physical side (mhd/boundary/phys.h:144-251): the cell is
             // written last by the side of the highest out-of-range axis that
             // is physical; its source is mirrored (reflect) or the boundary
@@ -117,11 +120,11 @@ __device__ __forceinline__ void load_cell(const MeshView<FT> &m, int b, const in
                     const int gd = side ? p[a] - m.n[a] : -1 - p[a];
                     if (kind == 3) {
                         q[a] = side ? m.n[a] - 1 - gd : gd;
-                        mflip = a;
+                        c.flip = a;
                     } else {
                         q[a] = side ? m.n[a] - 1 : 0;
-                        if (kind == 1) mclamp = 2 * a + side;
-                        if (kind == 4) fixd = true;
+                        if (kind == 1) c.clamp = 2 * a + side;
+                        if (kind == 4) c.fixd = true;
                     }
                 } else if (d[a] != 0 && ((g.phy >> (2 * a + side)) & 1)) {
                     q[a] = side ? m.n[a] - 1 : 0;
@@ -130,7 +133,7 @@ __device__ __forceinline__ void load_cell(const MeshView<FT> &m, int b, const in
                 out2 |= e[a] != 0;
             }
             if (out2) {
-                blk = g.nbr[nbr_dir(m, e)];
+                c.blk = g.nbr[nbr_dir(m, e)];
 #pragma unroll
                 for (int a = 0; a < 3; ++a) q[a] -= e[a] * m.n[a];
             }
@@ -138,42 +141,47 @@ __device__ __forceinline__ void load_cell(const MeshView<FT> &m, int b, const in
             for (int a = 0; a < 3; ++a) p[a] = q[a];
         }
     }
-    const FT *src = m.W + (size_t)blk * NV * m.ncell + cidx(m.n, p[0], p[1], p[2]);
 #pragma unroll
-    for (int v = 0; v < NV; ++v) w[v] = src[(size_t)v * m.ncell];
-    if constexpr (NV == 8) {
+    for (int a = 0; a < 3; ++a) c.p[a] = p[a];
+    return c;
+}
+
+// The boundary functor of a cell's source, on its primitives.
+template <class FT, int NV>
+__device__ __forceinline__ void cell_functor(const MeshView<FT> &m, const CellSrc &c, FT *w) {
 #pragma unroll
-        for (int a = 0; a < 3; ++a) {
-            if (mflip == a) {
-                w[MOM + a] = w[MOM + a] * -1;
+    for (int a = 0; a < 3; ++a) {
+        if (c.flip == a) {
+            w[MOM + a] = w[MOM + a] * -1;
+            if constexpr (NV == 8) {
 #pragma unroll
-                for (int c = 0; c < 3; ++c)
-                    if (c != a) w[BCC + c] = -w[BCC + c];
-            }
-            if (mclamp >= 0 && (mclamp >> 1) == a) {
-                const int side = mclamp & 1;
-                if (w[MOM + a] * (side ? -1 : 1) > 0) w[MOM + a] = 0;
-            }
-        }
-    }
-    if constexpr (NV == 5) {
-#pragma unroll
-        for (int a = 0; a < 3; ++a) {
-            if (flip == a) w[MOM + a] = w[MOM + a] * -1;
-            if ((clamp >> 1) == a && clamp >= 0) {
-                const int side = clamp & 1;
-                if (w[MOM + a] * (side ? -1 : 1) > 0) w[MOM + a] = 0;
+                for (int k = 0; k < 3; ++k)
+                    if (k != a) w[BCC + k] = -w[BCC + k];
             }
         }
+        if (c.clamp >= 0 && (c.clamp >> 1) == a) {
+            const int side = c.clamp & 1;
+            if (w[MOM + a] * (side ? -1 : 1) > 0) w[MOM + a] = 0;
+        }
     }
-    if (fixd) {             // hydro / mhd phys_functors.h fixed_t
+    if (c.fixd) {             // hydro / mhd phys_functors.h fixed_t
 #pragma unroll
         for (int v = 0; v < 5; ++v) w[v] = (FT)m.fix_w[v];
         if constexpr (NV == 8) {
 #pragma unroll
-            for (int c = 0; c < 3; ++c) w[BCC + c] = (FT)m.fix_b[c];
+            for (int k = 0; k < 3; ++k) w[BCC + k] = (FT)m.fix_b[k];
         }
     }
+}
+
+// Load the primitive vector of cell pin of block b.
+template <class FT, int NV>
+__device__ __forceinline__ void load_cell(const MeshView<FT> &m, int b, const int *pin, FT *w) {
+    const CellSrc c = cell_src<FT, NV>(m, b, pin);
+    const FT *src = m.W + (size_t)c.blk * NV * m.ncell + cidx(m.n, c.p[0], c.p[1], c.p[2]);
+#pragma unroll
+    for (int v = 0; v < NV; ++v) w[v] = src[(size_t)v * m.ncell];
+    cell_functor<FT, NV>(m, c, w);
 }
 
 // Normal face field of block b at face p (component c); transverse indices
@@ -255,58 +263,104 @@ __device__ __forceinline__ double block_min(double v) {
 }
 
 // ------------------------------------------------------------------- c2p
-// hydro/eos/adiabatic.h:211-259 and mhd/eos/adiabatic.h:127-235: primitives
-// with floors written back to the conserved slot, cell-centred B from the
-// face average, and at substep 0 the per-cell CFL dt reduced per workgroup.
+// Primitives of one cell (hydro/eos/adiabatic.h:211-259, mhd/eos/adiabatic.h
+// :127-235) from its conserved state in slot `slot`: healed values in cons,
+// prim, for MHD the cell-centred B from the face average and the squares
+// and face maxima that the CFL speeds use.  heal_rho: rho was raised to its
+// floor; moved: the energy that the slot should hold differs from what it
+// holds (the subtract / add round trip of the magnetic part, or a healed
+// pressure).  Returns c_s^2.
 template <class FT, bool MHD>
-__global__ void __launch_bounds__(kThreads) k_c2p(MeshView<FT> m, int step) {
-    if (m.ts[m.geo[blockIdx.y].grp].skip) return;
+__device__ __forceinline__ double cell_c2p(const MeshView<FT> &m, int b, int slot, int i, int j, int k,
+                                           double *cons, double *prim, double *bc, double *bc_2,
+                                           double *b_max, bool &heal_rho, bool &moved) {
+    const size_t c = cidx(m.n, i, j, k);
+    const double *U = m.U + ((size_t)b * 2 + slot) * 5 * m.ncell + c;
+#pragma unroll
+    for (int v = 0; v < 5; ++v) cons[v] = U[(size_t)v * m.ncell];
+    const EosPar e{m.gamma, m.cfl, m.d_floor, m.t_floor};
+    if constexpr (MHD) {
+        const double *BF = m.BF + ((size_t)b * 2 + slot) * 3 * m.nface;
+        double e_m(0);
+        const size_t f0 = fidx(m.n, i, j, k);
+        const size_t sh[3] = {1, (size_t)(m.n[0] + 1), (size_t)(m.n[0] + 1) * (m.n[1] + 1)};
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            // a thin (one-cell) axis has one face per cell, both sides
+            // of it (mhd/eos/adiabatic.h:164-177)
+            const double b_l = BF[(size_t)a * m.nface + f0];
+            const double b_r = m.n[a] < 2 ? b_l : BF[(size_t)a * m.nface + f0 + sh[a]];
+            const double bc_m = (b_l + b_r) / 2;
+            bc[a] = bc_m;
+            const double bcs2 = bc_m * bc_m;
+            e_m += bcs2;
+            bc_2[a] = bcs2;
+            b_max[a] = pmax(kfabs(b_l), kfabs(b_r));
+        }
+        e_m /= 2;
+        const double e_in = cons[ENE];
+        bool he;
+        cons[ENE] -= e_m;
+        const double cs2 = c2p(cons, prim, e, heal_rho, he);
+        cons[ENE] += e_m;
+        moved = cons[ENE] != e_in;
+        return cs2;
+    } else {
+        return c2p(cons, prim, e, heal_rho, moved);
+    }
+}
+
+// Global CFL reduction and the dt / t bookkeeping of redc_dt_start/finish
+// (mesh/cycle/cycle.cpp:77-115): p_dt = min(p_dt, CFL), dt_use clamped to
+// t_lim when topping up, t advanced, next seed = dt_use * dt_expand.
+__device__ __forceinline__ void take_dt(TimeState *ts, double cfl_dt) {
+    const double p = __builtin_fmin(cfl_dt, ts->p_dt);
+    const double dt_use = ts->top_up ? (p < ts->t_lim - ts->t ? p : ts->t_lim - ts->t) : p;
+    if (ts->top_up) {
+        const double tn = dt_use + ts->t;
+        ts->t = tn < ts->t_lim ? tn : ts->t_lim;
+    } else {
+        ts->t = dt_use + ts->t;
+    }
+    ts->dt_use = dt_use;
+    ts->p_dt = dt_use * ts->dt_expand;
+}
+
+// c2p of one substep: primitives with floors written back to the conserved
+// slot, and at substep 0 the per-cell CFL dt reduced per workgroup.
+//
+// FIN (substep 0 of small meshes): the workgroup that finishes last in its
+// time group also takes the group's dt, and the stop rule of cycle::step
+// (mesh/cycle/cycle.cpp:143-144) is evaluated here, so that no launch is
+// spent on either (k_cycle_begin and k_dt_finalize, together 6 to 9 us of a
+// cycle; on large meshes the arrivals would cost more than the launches).
+// arrived[g] counts the group's workgroups and is left at 0.
+template <class FT, bool MHD, bool FIN>
+__global__ void __launch_bounds__(kThreads) k_c2p(MeshView<FT> m, int step, const int *grp_first,
+                                                  int *arrived) {
+    const int b = blockIdx.y, grp = m.geo[b].grp;
+    TimeState *ts = m.ts + grp;
+    const bool skip = FIN ? ts->t >= ts->t_lim : ts->skip != 0;
+    if (!FIN && skip) return;
     constexpr int NV = MHD ? 8 : 5;
-    const int b = blockIdx.y;
     const size_t c = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     double dtc = (double)FLT_MAX;
-    if (c < m.ncell) {
+    if (c < m.ncell && !skip) {
         const int i = (int)(c % m.n[0]);
         const int j = (int)((c / m.n[0]) % m.n[1]);
         const int k = (int)(c / ((size_t)m.n[0] * m.n[1]));
+        double cons[5], prim[5], bc[3], bc_2[3], b_max[3];
+        bool heal_rho, moved;
+        const double cs2 = cell_c2p<FT, MHD>(m, b, step, i, j, k, cons, prim, bc, bc_2, b_max, heal_rho, moved);
         double *U = m.U + ((size_t)b * 2 + step) * 5 * m.ncell + c;
-        double cons[5], prim[5];
-#pragma unroll
-        for (int v = 0; v < 5; ++v) cons[v] = U[(size_t)v * m.ncell];
-        const EosPar e{m.gamma, m.cfl, m.d_floor, m.t_floor};
         const BlockGeo &g = m.geo[b];
         FT *W = m.W + (size_t)b * NV * m.ncell + c;
-        bool hr, he;
+        // the slot is written only where it does not hold the value already
+        if (moved) U[(size_t)ENE * m.ncell] = cons[ENE];
+        if (heal_rho) U[0] = cons[RHO];
+#pragma unroll
+        for (int v = 0; v < 5; ++v) W[(size_t)v * m.ncell] = (FT)prim[v];
         if constexpr (MHD) {
-            const double *BF = m.BF + ((size_t)b * 2 + step) * 3 * m.nface;
-            double bc[3], bc_2[3], b_max[3];
-            double e_m(0);
-            const size_t f0 = fidx(m.n, i, j, k);
-            const size_t sh[3] = {1, (size_t)(m.n[0] + 1), (size_t)(m.n[0] + 1) * (m.n[1] + 1)};
-#pragma unroll
-            for (int a = 0; a < 3; ++a) {
-                // a thin (one-cell) axis has one face per cell, both sides
-                // of it (mhd/eos/adiabatic.h:164-177)
-                const double b_l = BF[(size_t)a * m.nface + f0];
-                const double b_r = m.n[a] < 2 ? b_l : BF[(size_t)a * m.nface + f0 + sh[a]];
-                const double bc_m = (b_l + b_r) / 2;
-                bc[a] = bc_m;
-                const double bcs2 = bc_m * bc_m;
-                e_m += bcs2;
-                bc_2[a] = bcs2;
-                b_max[a] = pmax(kfabs(b_l), kfabs(b_r));
-            }
-            e_m /= 2;
-            const double e_in = cons[ENE];
-            cons[ENE] -= e_m;
-            c2p(cons, prim, e, hr, he);
-            cons[ENE] += e_m;
-            // the subtract / add round trip (and a healed pressure) can move
-            // the stored energy; where it did not, the slot already holds it
-            if (cons[ENE] != e_in) U[(size_t)ENE * m.ncell] = cons[ENE];
-            if (hr) U[0] = cons[RHO];
-#pragma unroll
-            for (int v = 0; v < 5; ++v) W[(size_t)v * m.ncell] = (FT)prim[v];
 #pragma unroll
             for (int a = 0; a < 3; ++a) W[(size_t)(BCC + a) * m.ncell] = (FT)bc[a];
             if (m.EC) {     // mhd/eos/adiabatic.h:214-219, from the stored values
@@ -318,20 +372,43 @@ __global__ void __launch_bounds__(kThreads) k_c2p(MeshView<FT> m, int step) {
                 E[2 * m.ncell] = B[0] * V[1] - B[1] * V[0];
             }
             if (step == 0)
-                dtc = std::is_same_v<FT, float> ? dt_mhd_mixed(prim, bc_2, b_max, g.dx, m.ndim, m.gamma, m.cfl)
-                                                : dt_mhd(prim, bc_2, b_max, g.dx, m.ndim, m.gamma, m.cfl);
-        } else {
-            const double cs2 = c2p(cons, prim, e, hr, he);
-            if (hr) U[0] = cons[RHO];
-            if (he) U[(size_t)ENE * m.ncell] = cons[ENE];
-#pragma unroll
-            for (int v = 0; v < 5; ++v) W[(size_t)v * m.ncell] = (FT)prim[v];
-            if (step == 0) dtc = dt_hydro(prim, cs2, g.dx, m.ndim, m.cfl);
+                dtc = std::is_same_v<FT, float>
+                          ? dt_mhd_mixed(prim, bc_2, b_max, g.dx, m.ndim, m.gamma, m.cfl)
+                          : dt_mhd(prim, bc_2, b_max, g.dx, m.ndim, m.gamma, m.cfl);
+        } else if (step == 0) {
+            dtc = dt_hydro(prim, cs2, g.dx, m.ndim, m.cfl);
         }
     }
-    if (step == 0) {
+    if constexpr (!FIN) {
+        if (step == 0) {
+            const double r = block_min(dtc);
+            if (threadIdx.x == 0) m.dt_part[(size_t)b * gridDim.x + blockIdx.x] = r;
+        }
+    } else {
         const double r = block_min(dtc);
-        if (threadIdx.x == 0) m.dt_part[(size_t)blockIdx.y * gridDim.x + blockIdx.x] = r;
+        const int first = grp_first[grp], last = grp_first[grp + 1];
+        __shared__ bool s_last;
+        if (threadIdx.x == 0) {
+            __hip_atomic_store(m.dt_part + (size_t)b * gridDim.x + blockIdx.x, r, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+            const int n = __hip_atomic_fetch_add(arrived + grp, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+            s_last = n + 1 == (last - first) * (int)gridDim.x;
+        }
+        __syncthreads();
+        if (!s_last) return;
+        double v = (double)FLT_MAX;
+        for (size_t i = (size_t)first * gridDim.x + threadIdx.x; i < (size_t)last * gridDim.x; i += kThreads)
+            v = pmin(v, __hip_atomic_load(m.dt_part + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+        __syncthreads();                     // block_min's scratch is read above by thread 0
+        v = block_min(v);
+        if (threadIdx.x == 0) {
+            ts->skip = skip ? 1 : 0;
+            if (!skip) {
+                ts->cycles += 1;
+                take_dt(ts, v);
+            }
+            __hip_atomic_store(arrived + grp, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
     }
 }
 
