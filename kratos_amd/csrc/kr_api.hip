@@ -4,6 +4,7 @@
 #include "../../include/kratos_amd.h"
 #include "kr_fused.h"
 #include "kr_fused_hydro.h"
+#include "kr_pack.h"
 #include "kr_plane.h"
 #include "kr_smr.h"
 #include "kr_sweep64.h"
@@ -161,6 +162,10 @@ unsigned z_ranges(size_t wgs, int ncu, int per_cu, int nz, double lat) {
     return best;
 }
 
+// Doubles of one half of the transfer buffer (1 MiB): while the host copies
+// one half, the GPU fills the other.
+constexpr size_t kPinDoubles = 131072;
+
 // Most c2p workgroups of a mesh whose last one takes the dt (FIN): up to
 // there the arrivals cost less than the two launches they replace (32^3: 128
 // workgroups, 92 -> 85 us a cycle).
@@ -269,7 +274,11 @@ struct kr_ctx {
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     kr_stats stats{};
     float tune_ms[kNumSweepVariants] = {0};
-    std::vector<double> stage;   // host staging for packing
+    // page-locked host memory that the kernels address: two halves of
+    // kPinDoubles for a transfer, and two snapshots of the time states
+    double *pin = nullptr;
+    TimeState *hts = nullptr;
+    hipEvent_t pin_ev[2] = {nullptr, nullptr};
 
     template <class FT> MeshView<FT> view() const {
         MeshView<FT> m{};
@@ -312,6 +321,10 @@ void release(kr_ctx *c) {
                     c->d_pure, c->d_pfill, c->d_sweep, c->d_items, c->d_nitems, c->arrived};
     for (void *p : bufs)
         if (p) (void)hipFree(p);
+    if (c->pin) (void)hipHostFree(c->pin);
+    if (c->hts) (void)hipHostFree(c->hts);
+    c->pin = nullptr;
+    c->hts = nullptr;
     c->d_table = nullptr;
     c->d_fill[0] = c->d_fill[1] = nullptr;
     c->d_pfill = nullptr;
@@ -761,6 +774,8 @@ void commit(kr_ctx *c) {
     std::vector<TimeState> tsv(c->ngrp, ts);
     c->ts = dalloc<TimeState>(c->ngrp);
     KR_HIP(hipMemcpy(c->ts, tsv.data(), c->ngrp * sizeof(ts), hipMemcpyHostToDevice));
+    KR_HIP(hipHostMalloc((void **)&c->hts, 2 * c->ngrp * sizeof(TimeState), hipHostMallocDefault));
+    KR_HIP(hipHostMalloc((void **)&c->pin, 2 * kPinDoubles * sizeof(double), hipHostMallocDefault));
     c->grp_first = dalloc<int>(c->ngrp + 1);
     KR_HIP(hipMemcpy(c->grp_first, first.data(), (c->ngrp + 1) * sizeof(int), hipMemcpyHostToDevice));
 
@@ -798,6 +813,8 @@ void commit(kr_ctx *c) {
     c->stats.n_cells = (long long)(nb * c->ncell);
     // 5 state passes per Heun cycle of (5 conserved + 3 face-B) FP64 values
     c->stats.alg_bytes_per_cell_update = 5.0 * (5 + (c->mhd ? 3 : 0)) * 8.0;
+    // the fills above run on the default stream, everything later on c->stream
+    KR_HIP(hipStreamSynchronize(nullptr));
     c->committed = true;
 }
 
@@ -1190,17 +1207,22 @@ template <class F> int guarded(kr_ctx *c, F &&f) {
     }
 }
 
-TimeState read_ts(kr_ctx *c, int g = 0) {
-    TimeState ts{};
-    KR_HIP(hipMemcpy(&ts, c->ts + g, sizeof(ts), hipMemcpyDeviceToHost));
-    return ts;
+// Snapshot `which` (0 or 1) of every time state, in stream order.
+void report(kr_ctx *c, int which) {
+    hipLaunchKernelGGL(k_report, dim3(ceil_div(c->ngrp, kThreads)), dim3(kThreads), 0, c->stream,
+                       (const TimeState *)c->ts, c->ngrp, c->hts + (size_t)which * c->ngrp);
+    KR_HIP(hipGetLastError());
 }
-
+std::vector<TimeState> reported(const kr_ctx *c, int which) {
+    const TimeState *t = c->hts + (size_t)which * c->ngrp;
+    return std::vector<TimeState>(t, t + c->ngrp);
+}
 std::vector<TimeState> read_all_ts(kr_ctx *c) {
-    std::vector<TimeState> v(c->ngrp);
-    KR_HIP(hipMemcpy(v.data(), c->ts, c->ngrp * sizeof(TimeState), hipMemcpyDeviceToHost));
-    return v;
+    report(c, 0);
+    KR_HIP(hipStreamSynchronize(c->stream));
+    return reported(c, 0);
 }
+TimeState read_ts(kr_ctx *c, int g = 0) { return read_all_ts(c)[g]; }
 
 // cycles run by the slowest-stopping group between two snapshots, and
 // whether every group has reached t_lim
@@ -1235,75 +1257,92 @@ double *noalloc_scratch() {
 
 namespace {
 
+HostShape host_shape(const kr_ctx *c, bool bf) {
+    HostShape h{};
+    size_t nf = 1;
+    for (int a = 0; a < 3; ++a) {
+        h.n[a] = c->n[a];
+        // n + (n > 1) faces per axis plus two ghost layers each side
+        // (mhd/types/fld_data.cpp:18-26); a thin axis has one
+        h.N[a] = c->n[a] + (c->n[a] > 1) + 4;
+        nf *= (size_t)h.N[a];
+    }
+    h.nvar = c->mhd ? 8 : 5;
+    h.nu = c->ncell * h.nvar;
+    h.nbf = bf ? nf * 3 : 0;
+    return h;
+}
+
+// [i0, i0 + count) of the host arrays (u, then bf) against one buffer.
+template <class F> void each_part(const HostShape &h, size_t i0, size_t count, F &&f) {
+    const size_t i1 = i0 + count;
+    if (i0 < h.nu) f(false, i0, std::min(i1, h.nu) - i0, (size_t)0);
+    if (i1 > h.nu) {
+        const size_t k = std::max(i0, h.nu);
+        f(true, k - h.nu, i1 - k, k - i0);
+    }
+}
+
+// Runs the chunks of a transfer of `total` doubles over the two halves of
+// the buffer: before(k) is host work on half k % 2 before its kernel, after(k)
+// host work once that kernel has finished.
+template <class Before, class Kernel, class After>
+void transfer(kr_ctx *c, size_t total, Before &&before, Kernel &&kernel, After &&after) {
+    const size_t n = ceil_div(total, kPinDoubles);
+    for (size_t k = 0; k <= n; ++k) {
+        if (k < n) {
+            const size_t i0 = k * kPinDoubles, cnt = std::min(kPinDoubles, total - i0);
+            before(i0, cnt, c->pin + (k & 1) * kPinDoubles);
+            kernel(i0, cnt, c->pin + (k & 1) * kPinDoubles);
+            KR_HIP(hipGetLastError());
+            if (n > 1) KR_HIP(hipEventRecord(c->pin_ev[k & 1], c->stream));
+        }
+        if (k > 0) {
+            const size_t i0 = (k - 1) * kPinDoubles, cnt = std::min(kPinDoubles, total - i0);
+            if (n > 1) KR_HIP(hipEventSynchronize(c->pin_ev[(k - 1) & 1]));
+            else KR_HIP(hipStreamSynchronize(c->stream));
+            after(i0, cnt, c->pin + ((k - 1) & 1) * kPinDoubles);
+        }
+    }
+}
+
 // One block of n_cell_block cells from the reference's host layout into
 // slot 0 of the pools: u_aos interior cells, bf_aos the ghosted face array.
 void upload_one(kr_ctx *c, size_t b, const double *u_aos, const double *bf_aos) {
-    const int nvar = c->mhd ? 8 : 5;
-    std::vector<double> &s = c->stage;
-    s.assign(5 * c->ncell, 0.0);
-    for (size_t cc = 0; cc < c->ncell; ++cc)
-        for (int v = 0; v < 5; ++v) s[v * c->ncell + cc] = u_aos[cc * nvar + v];
-    KR_HIP(hipMemcpy(c->U + b * 2 * 5 * c->ncell, s.data(), 5 * c->ncell * sizeof(double),
-                     hipMemcpyHostToDevice));
-    if (c->mhd) {
-        // host face array: n + (n > 1) faces per axis plus two ghost layers
-        // each side (mhd/types/fld_data.cpp:18-26); a thin axis has one
-        const int nf[3] = {c->n[0] + (c->n[0] > 1), c->n[1] + (c->n[1] > 1),
-                           c->n[2] + (c->n[2] > 1)};
-        const int N0 = nf[0] + 4, N1 = nf[1] + 4;
-        s.assign(3 * c->nface, 0.0);
-        for (int k = 0; k < nf[2]; ++k)
-            for (int j = 0; j < nf[1]; ++j)
-                for (int i = 0; i < nf[0]; ++i) {
-                    const size_t src = ((size_t)((k + 2) * N1 + (j + 2)) * N0 + (i + 2)) * 3;
-                    const size_t f = ((size_t)k * (c->n[1] + 1) + j) * (c->n[0] + 1) + i;
-                    for (int a = 0; a < 3; ++a) s[a * c->nface + f] = bf_aos[src + a];
-                }
-        KR_HIP(hipMemcpy(c->BF + b * 2 * 3 * c->nface, s.data(), 3 * c->nface * sizeof(double),
-                         hipMemcpyHostToDevice));
-    }
+    const HostShape h = host_shape(c, c->mhd);
+    double *U = c->U + b * 2 * 5 * c->ncell;
+    double *BF = c->mhd ? c->BF + b * 2 * 3 * c->nface : nullptr;
+    transfer(
+        c, h.nu + h.nbf,
+        [&](size_t i0, size_t cnt, double *buf) {
+            each_part(h, i0, cnt, [&](bool bf, size_t at, size_t n, size_t off) {
+                std::memcpy(buf + off, (bf ? bf_aos : u_aos) + at, n * sizeof(double));
+            });
+        },
+        [&](size_t i0, size_t cnt, const double *buf) {
+            hipLaunchKernelGGL(k_unpack, dim3(ceil_div(cnt, kThreads)), dim3(kThreads), 0, c->stream, h, U,
+                               BF, c->ncell, c->nface, i0, cnt, buf);
+        },
+        [](size_t, size_t, const double *) {});
 }
 
 // One block of n_cell_block cells back into the reference's host layout
 // (cell-centred B from the face average; faces with zero ghost layers).
 void download_one(kr_ctx *c, size_t b, double *u_aos, double *bf_aos) {
-    const int nvar = c->mhd ? 8 : 5;
-    std::vector<double> s(5 * c->ncell);
-    KR_HIP(hipMemcpy(s.data(), c->U + b * 2 * 5 * c->ncell, 5 * c->ncell * sizeof(double),
-                     hipMemcpyDeviceToHost));
-    for (size_t cc = 0; cc < c->ncell; ++cc)
-        for (int v = 0; v < 5; ++v) u_aos[cc * nvar + v] = s[v * c->ncell + cc];
-    if (c->mhd) {
-        std::vector<double> f(3 * c->nface);
-        KR_HIP(hipMemcpy(f.data(), c->BF + b * 2 * 3 * c->nface, 3 * c->nface * sizeof(double),
-                         hipMemcpyDeviceToHost));
-        // a thin axis has one face, both sides of the cell
-        const size_t sh[3] = {c->n[0] > 1 ? (size_t)1 : 0,
-                              c->n[1] > 1 ? (size_t)(c->n[0] + 1) : 0,
-                              c->n[2] > 1 ? (size_t)(c->n[0] + 1) * (c->n[1] + 1) : 0};
-        for (int k = 0; k < c->n[2]; ++k)
-            for (int j = 0; j < c->n[1]; ++j)
-                for (int i = 0; i < c->n[0]; ++i) {
-                    const size_t cc = ((size_t)k * c->n[1] + j) * c->n[0] + i;
-                    const size_t f0 = ((size_t)k * (c->n[1] + 1) + j) * (c->n[0] + 1) + i;
-                    for (int a = 0; a < 3; ++a)
-                        u_aos[cc * nvar + BCC + a] =
-                            (f[a * c->nface + f0] + f[a * c->nface + f0 + sh[a]]) / 2;
-                }
-        if (bf_aos) {
-            const int nf[3] = {c->n[0] + (c->n[0] > 1), c->n[1] + (c->n[1] > 1),
-                               c->n[2] + (c->n[2] > 1)};
-            const int N0 = nf[0] + 4, N1 = nf[1] + 4, N2 = nf[2] + 4;
-            std::memset(bf_aos, 0, (size_t)N0 * N1 * N2 * 3 * sizeof(double));
-            for (int k = 0; k < nf[2]; ++k)
-                for (int j = 0; j < nf[1]; ++j)
-                    for (int i = 0; i < nf[0]; ++i) {
-                        const size_t dst = ((size_t)((k + 2) * N1 + (j + 2)) * N0 + (i + 2)) * 3;
-                        const size_t f0 = ((size_t)k * (c->n[1] + 1) + j) * (c->n[0] + 1) + i;
-                        for (int a = 0; a < 3; ++a) bf_aos[dst + a] = f[a * c->nface + f0];
-                    }
-        }
-    }
+    const HostShape h = host_shape(c, c->mhd && bf_aos);
+    const double *U = c->U + b * 2 * 5 * c->ncell;
+    const double *BF = c->mhd ? c->BF + b * 2 * 3 * c->nface : nullptr;
+    transfer(
+        c, h.nu + h.nbf, [](size_t, size_t, const double *) {},
+        [&](size_t i0, size_t cnt, double *buf) {
+            hipLaunchKernelGGL(k_pack, dim3(ceil_div(cnt, kThreads)), dim3(kThreads), 0, c->stream, h, U,
+                               BF, c->ncell, c->nface, i0, cnt, buf);
+        },
+        [&](size_t i0, size_t cnt, const double *buf) {
+            each_part(h, i0, cnt, [&](bool bf, size_t at, size_t n, size_t off) {
+                std::memcpy((bf ? bf_aos : u_aos) + at, buf + off, n * sizeof(double));
+            });
+        });
 }
 
 // Host arrays of a block of 2n cells per axis <-> its octant o's arrays of
@@ -1388,6 +1427,7 @@ int kr_create(const kr_config *cfg, kr_ctx **out) {
         KR_HIP(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
         KR_HIP(hipEventCreate(&c->ev0));
         KR_HIP(hipEventCreate(&c->ev1));
+        for (int k = 0; k < 2; ++k) KR_HIP(hipEventCreateWithFlags(&c->pin_ev[k], hipEventDisableTiming));
         return KR_OK;
     });
     if (rc != KR_OK) {
@@ -1503,7 +1543,7 @@ int kr_download(kr_ctx *c, int id, double *u_aos, double *bf_aos) {
 int kr_step(kr_ctx *c, double *dt_taken) {
     return guarded(c, [&] {
         commit(c);
-        const auto before = read_all_ts(c);
+        report(c, 0);
         KR_HIP(hipEventRecord(c->ev0, c->stream));
         if (tuning(c)) {
             tune_cycle(c);
@@ -1512,10 +1552,11 @@ int kr_step(kr_ctx *c, double *dt_taken) {
             L.cycle();
         }
         KR_HIP(hipEventRecord(c->ev1, c->stream));
+        report(c, 1);
         KR_HIP(hipStreamSynchronize(c->stream));
         float ms = 0;
         KR_HIP(hipEventElapsedTime(&ms, c->ev0, c->ev1));
-        const auto after = read_all_ts(c);
+        const auto before = reported(c, 0), after = reported(c, 1);
         c->stats.gpu_ms = ms;
         fill_tile_stats(c);
         c->stats.cycles = cycles_between(before, after);
@@ -1530,6 +1571,7 @@ int kr_advance(kr_ctx *c, int n_cycles, int *n_done) {
         commit(c);
         if (n_cycles < 0) throw std::invalid_argument("n_cycles < 0");
         const auto before = read_all_ts(c);
+        auto after = before;
         double ms_tot = 0;
         int left = n_cycles;
         bool done = all_done(before);
@@ -1543,7 +1585,8 @@ int kr_advance(kr_ctx *c, int n_cycles, int *n_done) {
             KR_HIP(hipEventElapsedTime(&ms, c->ev0, c->ev1));
             ms_tot += ms;
             --left;
-            done = all_done(read_all_ts(c));
+            after = read_all_ts(c);
+            done = all_done(after);
         }
         if (left > 0 && !done && !c->graph) {
             hipGraph_t g;
@@ -1561,14 +1604,15 @@ int kr_advance(kr_ctx *c, int n_cycles, int *n_done) {
             KR_HIP(hipEventRecord(c->ev0, c->stream));
             for (int i = 0; i < chunk; ++i) KR_HIP(hipGraphLaunch(c->graph, c->stream));
             KR_HIP(hipEventRecord(c->ev1, c->stream));
+            report(c, 1);
             KR_HIP(hipStreamSynchronize(c->stream));
             float ms = 0;
             KR_HIP(hipEventElapsedTime(&ms, c->ev0, c->ev1));
             ms_tot += ms;
             left -= chunk;
-            if (left > 0) done = all_done(read_all_ts(c));
+            after = reported(c, 1);
+            done = all_done(after);
         }
-        const auto after = read_all_ts(c);
         c->stats.gpu_ms = ms_tot;
         fill_tile_stats(c);
         c->stats.cycles = cycles_between(before, after);
@@ -1726,6 +1770,8 @@ void kr_destroy(kr_ctx *c) {
     release(c);
     if (c->ev0) (void)hipEventDestroy(c->ev0);
     if (c->ev1) (void)hipEventDestroy(c->ev1);
+    for (int k = 0; k < 2; ++k)
+        if (c->pin_ev[k]) (void)hipEventDestroy(c->pin_ev[k]);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
 }
