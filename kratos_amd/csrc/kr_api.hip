@@ -4,10 +4,10 @@
 #include "../../include/kratos_amd.h"
 #include "kr_fused.h"
 #include "kr_fused_hydro.h"
+#include "kr_march.h"
 #include "kr_pack.h"
 #include "kr_plane.h"
 #include "kr_smr.h"
-#include "kr_sweep64.h"
 #include "kr_sweep_mx.h"
 
 #include <hip/hip_runtime.h>
@@ -184,14 +184,16 @@ constexpr int kAdvanceChunk = 64;
 enum SweepKernel {
     SK_SWEEP = 0,   // k_sweep (mixed MHD with physical sides or refinement), k_sweep_hyd
     SK_MX = 1,      // k_sweep_mx (mixed MHD, one level, periodic)
-    SK_64 = 2,      // k_sweep64 (FP64 MHD)
+    SK_64 = 2,      // k_march (FP64 MHD)
     SK_64_NARROW = 3,   // ... where no wider tile fits the blocks
-    SK_64_TILE = 4      // ... when kr_config.tile asks for it: never the fastest
+    SK_64_TILE = 4,     // ... when kr_config.tile asks for it: never the fastest
+    SK_ODD = 5,     // k_march (mixed MHD, blocks that 8x8 tiles do not divide)
+    SK_STAGED = 6   // the staged kernels: on odd blocks and refined meshes they may win
 };
 struct SweepVariant {
     int tx, ty, nt, waves, kernel;
 };
-// k_sweep64: a 16x8 tile's solves of a plane fill 256 threads twice or 512
+// k_march: a 16x8 tile's solves of a plane fill 256 threads twice or 512
 // once.  Two workgroups of 256 overlap on a compute unit and win where the
 // tiles fill the GPU (128^3 in 32^3 blocks: 0.52 against 0.60 ms a launch);
 // one of 512 takes half as long over a plane where they do not (64^3: 93
@@ -204,6 +206,7 @@ constexpr SweepVariant kSweepVariants[] = {
     {16, 16, 512, 1, SK_MX},    {8, 8, 192, 1, SK_MX},     {32, 8, 512, 1, SK_64},
     {16, 8, 512, 1, SK_64},     {16, 8, 256, 1, SK_64},    {8, 8, 320, 1, SK_64},
     {16, 16, 512, 1, SK_64_TILE}, {8, 8, 192, 1, SK_64_NARROW},
+    {16, 8, 256, 1, SK_ODD},    {8, 8, 192, 1, SK_ODD},   {0, 0, 0, 1, SK_STAGED},
 };
 constexpr int kNumSweepVariants = sizeof(kSweepVariants) / sizeof(kSweepVariants[0]);
 
@@ -280,6 +283,9 @@ struct kr_ctx {
     TimeState *hts = nullptr;
     hipEvent_t pin_ev[2] = {nullptr, nullptr};
 
+    // the fused kernels run (or, while tuning, the candidate at hand is one)
+    bool fused_now() const { return fused && kSweepVariants[variant].kernel != SK_STAGED; }
+
     template <class FT> MeshView<FT> view() const {
         MeshView<FT> m{};
         for (int a = 0; a < 3; ++a) m.n[a] = n[a];
@@ -302,7 +308,7 @@ struct kr_ctx {
         m.W = (FT *)W;
         for (int a = 0; a < 3; ++a) m.F[a] = (FT *)F[a];
         m.EE = (FT *)EE;
-        m.EC = (FT *)EC;
+        m.EC = !fused_now() || (smr && prod < 0) ? (FT *)EC : nullptr;
         m.geo = geo;
         m.ts = ts;
         m.dt_part = dt_part;
@@ -687,21 +693,35 @@ void commit(kr_ctx *c) {
                                     "physical sides");
     if (!(c->smr && phys_sides) && c->cfg.kernel_path != KR_PATH_STAGED) {
         const int tx = c->cfg.tile[0], ty = c->cfg.tile[1], tw = c->cfg.tile[2];
-        const bool mxmesh = c->mixed && c->mhd && !c->smr && !phys_sides;
+        // Blocks that a tile does not divide: path auto takes them too (a tile
+        // moved back into the block), except the mixed MHD kernels k_sweep and
+        // k_sweep_mx, which want whole tiles; where not even 8x8 divides the
+        // block, k_march runs the mixed form with the staged kernels' rounding.
+        const bool odd = c->n[0] % 8 != 0 || c->n[1] % 8 != 0;
+        const bool any_size = c->cfg.kernel_path == KR_PATH_AUTO;
+        const bool f64 = c->mhd && !c->mixed, f32 = c->mhd && c->mixed;
+        const bool mxmesh = f32 && !c->smr && !phys_sides && !odd;
         c->candidates.clear();
         for (int v = 0; v < kNumSweepVariants; ++v) {
             const SweepVariant &sv = kSweepVariants[v];
-            const bool f64 = c->mhd && !c->mixed;
-            if ((sv.kernel == SK_MX) && !mxmesh) continue;
+            if (sv.kernel == SK_MX && !mxmesh) continue;
             if (mxmesh && sv.kernel == SK_SWEEP && !(tx && tw > 1)) continue;
-            if (f64 != (sv.kernel >= SK_64)) continue;
+            if (f64 != (sv.kernel >= SK_64 && sv.kernel <= SK_64_TILE) && sv.kernel != SK_STAGED) continue;
+            if (sv.kernel == SK_STAGED) {
+                // equal bit for bit to every candidate here but k_sweep's
+                if (any_size && !tx && !tw && (odd || (c->smr && !f32)) && !c->candidates.empty())
+                    c->candidates.push_back(v);
+                continue;
+            }
+            if ((f32 && odd) != (sv.kernel == SK_ODD)) continue;
             if (sv.kernel == SK_64_TILE && !tx) continue;
-            if (sv.kernel == SK_64_NARROW && c->n[0] % 16 == 0) continue;
+            if (sv.kernel == SK_64_NARROW && c->n[0] >= 16) continue;
             if (tx && (sv.tx != tx || sv.ty != ty)) continue;
             if (tw && sv.waves != tw) continue;
             if (sv.waves > 1 && (!c->mixed || !c->mhd)) continue;
-            if (c->n[0] % sv.tx == 0 && c->n[1] % sv.ty == 0 && c->n[2] >= 4)
-                c->candidates.push_back(v);
+            const bool whole = c->n[0] % sv.tx == 0 && c->n[1] % sv.ty == 0;
+            const bool fits = any_size && sv.waves == 1 && (!f32 || odd) && c->n[0] >= sv.tx && c->n[1] >= sv.ty;
+            if ((whole || fits) && c->n[2] >= 4) c->candidates.push_back(v);
         }
         if (c->candidates.empty() && c->cfg.kernel_path == KR_PATH_FUSED)
             throw std::invalid_argument("no fused tile fits the block shape");
@@ -807,7 +827,8 @@ void commit(kr_ctx *c) {
         c->tune_next = 0;
     }
     // cell-centred E for the staged EMF kernel, when it runs
-    if (c->mhd && !c->plane && (!c->fused || (c->smr && c->prod < 0)))
+    const bool may_stage = !c->fused || kSweepVariants[c->candidates.back()].kernel == SK_STAGED;
+    if (c->mhd && !c->plane && (may_stage || (c->smr && c->prod < 0)))
         KR_HIP(hipMalloc(&c->EC, nb * 3 * c->ncell * fs));
     c->stats.n_blocks = (int)nb;
     c->stats.n_cells = (long long)(nb * c->ncell);
@@ -822,18 +843,14 @@ void commit(kr_ctx *c) {
 struct Launcher {
     kr_ctx *c;
     bool prof = false;   // events around every launch
-    bool tune = false;   // events around the fused stage-kernel launches only
-    bool again = false;  // the stage's fused launch may run twice (substep 0 reads slot 0 only)
+    bool tune = false;   // events around each stage past its c2p
     std::vector<std::pair<int, std::pair<hipEvent_t, hipEvent_t>>> evs;
 
-    template <class F> void run(int kind, F &&f, bool sweep_launch = false) {
-        if (!prof && !(tune && sweep_launch)) {
-            f();
-            return;
-        }
-        // a kernel's first launch also loads its code (3x the time of the next
-        // one on a small mesh): tuning times the next
-        if (tune && again) f();
+    template <class F> void run(int kind, F &&f) {
+        if (!prof) f();
+        else timed(kind, f);
+    }
+    template <class F> void timed(int kind, F &&f) {
         hipEvent_t a, b;
         KR_HIP(hipEventCreate(&a));
         KR_HIP(hipEventCreate(&b));
@@ -865,7 +882,7 @@ struct Launcher {
     template <class K, class FT>
     void launch(K fn, const MeshView<FT> &m, int step, int variant, int tx, int ty, int threads,
                 unsigned nb, double lat) {
-        const unsigned nt = (unsigned)((c->n[0] / tx) * (c->n[1] / ty));
+        const unsigned nt = (unsigned)(march_tiles(c->n[0], tx) * march_tiles(c->n[1], ty));
         const unsigned kz = ranges(fn, variant, threads, nt, nb, lat);
         hipLaunchKernelGGL(fn, dim3(nt, nb, kz), dim3(threads), 0, c->stream, m, step);
     }
@@ -875,16 +892,20 @@ struct Launcher {
         launch(c->npfill ? k_sweep<TX, TY, NT, W, PROD, true> : k_sweep<TX, TY, NT, W, PROD, false>, m,
                step, PROD ? kNumSweepVariants : c->variant, TX, TY, NT, nb, kLatMhdMixed);
     }
-    template <int TX, int TY, int NT, int PROD = 0>
-    void sweep64_t(const MeshView<double> &m, int step, unsigned nb) {
-        launch(c->npfill ? k_sweep64<TX, TY, NT, PROD, true> : k_sweep64<TX, TY, NT, PROD, false>, m, step,
-               PROD ? kNumSweepVariants : c->variant, TX, TY, NT, nb, kLatMhd64);
+    template <class FT, int TX, int TY, int NT, int PROD = 0>
+    void march_t(const MeshView<FT> &m, int step, unsigned nb) {
+        // FP32: the build with the rules of physical sides everywhere (they do
+        // nothing on a periodic mesh): it rounds as the staged kernels do
+        launch(c->npfill || std::is_same_v<FT, float> ? k_march<FT, TX, TY, NT, PROD, true>
+                                                      : k_march<FT, TX, TY, NT, PROD, false>,
+               m, step, PROD ? kNumSweepVariants : c->variant, TX, TY, NT, nb,
+               std::is_same_v<FT, double> ? kLatMhd64 : kLatMhdMixed);
     }
     // FP64: fluxes and edge EMFs of the listed blocks into F / EE (no update)
     void sweep_prod(const MeshView<double> &m, int step, unsigned nb) {
-        if (c->prod == 0) sweep64_t<16, 8, 256, 1>(m, step, nb);
-        else if (nb * (unsigned)((c->n[0] / 8) * (c->n[1] / 8)) <= 512) sweep64_t<8, 8, 320, 1>(m, step, nb);
-        else sweep64_t<8, 8, 192, 1>(m, step, nb);
+        if (c->prod == 0) march_t<double, 16, 8, 256, 1>(m, step, nb);
+        else if (nb * (unsigned)((c->n[0] / 8) * (c->n[1] / 8)) <= 512) march_t<double, 8, 8, 320, 1>(m, step, nb);
+        else march_t<double, 8, 8, 192, 1>(m, step, nb);
     }
     // mixed: the full form on the first rows, the producer form on the others
     void sweep_both(const MeshView<float> &m, int step, unsigned nb) {
@@ -919,17 +940,19 @@ struct Launcher {
         case 7: sweep_mx_t<16, 8, 256>(m, step, nb); break;
         case 8: sweep_mx_t<32, 8, 512>(m, step, nb); break;
         case 9: sweep_mx_t<16, 16, 512>(m, step, nb); break;
-        default: sweep_mx_t<8, 8, 192>(m, step, nb); break;
+        case 10: sweep_mx_t<8, 8, 192>(m, step, nb); break;
+        case 17: march_t<float, 16, 8, 256>(m, step, nb); break;
+        default: march_t<float, 8, 8, 192>(m, step, nb); break;
         }
     }
     void sweep(const MeshView<double> &m, int step, int variant, unsigned nb) {
         switch (variant) {
-        case 11: sweep64_t<32, 8, 512>(m, step, nb); break;
-        case 12: sweep64_t<16, 8, 512>(m, step, nb); break;
-        case 13: sweep64_t<16, 8, 256>(m, step, nb); break;
-        case 14: sweep64_t<8, 8, 320>(m, step, nb); break;
-        case 15: sweep64_t<16, 16, 512>(m, step, nb); break;
-        default: sweep64_t<8, 8, 192>(m, step, nb); break;
+        case 11: march_t<double, 32, 8, 512>(m, step, nb); break;
+        case 12: march_t<double, 16, 8, 512>(m, step, nb); break;
+        case 13: march_t<double, 16, 8, 256>(m, step, nb); break;
+        case 14: march_t<double, 8, 8, 320>(m, step, nb); break;
+        case 15: march_t<double, 16, 16, 512>(m, step, nb); break;
+        default: march_t<double, 8, 8, 192>(m, step, nb); break;
         }
     }
     // Ensembles: the stage's work list (the tiles of the boxes still
@@ -970,7 +993,6 @@ struct Launcher {
     }
 
     template <class FT, bool MHD> void stage(int step) {
-        again = step == 0;
         const MeshView<FT> m = c->view<FT>();
         const unsigned nb = (unsigned)c->descs.size();
         const dim3 blk(kThreads);
@@ -993,8 +1015,23 @@ struct Launcher {
             run(KR_K_UPDATE, [&] { plane<FT, MHD, false>(m, step, nb); });
             return;
         }
+        if (!tune) {
+            solve<FT, MHD>(m, step, nb);
+            return;
+        }
+        // a kernel's first launch also loads its code (3x the time of the next
+        // one on a small mesh).  Substep 0 only reads slot 0 past its c2p, so
+        // tuning runs it twice and times the second.
+        if (step == 0) solve<FT, MHD>(m, step, nb);
+        timed(KR_K_UPDATE, [&] { solve<FT, MHD>(m, step, nb); });
+    }
+
+    // A stage past its c2p: fluxes, EMFs and the update.
+    template <class FT, bool MHD> void solve(const MeshView<FT> &m, int step, unsigned nb) {
+        const dim3 blk(kThreads);
+        const bool fused = c->fused_now();
         constexpr int NV = MHD ? 8 : 5;
-        if (c->fused && !c->smr) {
+        if (fused && !c->smr) {
             if (c->npfill)                  // physical-side halos (accounted as c2p)
                 run(KR_K_C2P, [&] {
                     const size_t mx = 4 * (size_t)std::max(c->n[0] * c->n[1],
@@ -1003,9 +1040,9 @@ struct Launcher {
                                        dim3(256), 0, c->stream, m, (const int4 *)c->d_pfill);
                 });
             if constexpr (MHD)
-                run(KR_K_UPDATE, [&] { sweep(m, step, c->variant, nb); }, true);
+                run(KR_K_UPDATE, [&] { sweep(m, step, c->variant, nb); });
             else
-                run(KR_K_UPDATE, [&] { sweep_hyd<FT>(m, step, c->variant, nb); }, true);
+                run(KR_K_UPDATE, [&] { sweep_hyd<FT>(m, step, c->variant, nb); });
             return;
         }
         if (c->smr) {                       // halo where levels meet (accounted as c2p)
@@ -1028,7 +1065,7 @@ struct Launcher {
         // kernel the blocks that touch another level (the rest run fused)
         MeshView<FT> ms = m;
         unsigned ns = nb;
-        if (c->smr && c->fused) {
+        if (c->smr && fused) {
             bool both = false;
             if constexpr (MHD && std::is_same_v<FT, float>)
                 if (c->prod >= 0) {
@@ -1038,23 +1075,22 @@ struct Launcher {
                     mb.blist = c->d_sweep;
                     mb.nfull = c->npure;
                     run(KR_K_UPDATE,
-                        [&] { sweep_both(mb, step, (unsigned)(c->npure + c->nxblk)); }, true);
+                        [&] { sweep_both(mb, step, (unsigned)(c->npure + c->nxblk)); });
                     both = true;
                 }
             if (!both && c->npure) {
                 MeshView<FT> mp = m;
                 mp.blist = c->d_pure;
                 if constexpr (MHD)
-                    run(KR_K_UPDATE, [&] { sweep(mp, step, c->variant, (unsigned)c->npure); }, true);
+                    run(KR_K_UPDATE, [&] { sweep(mp, step, c->variant, (unsigned)c->npure); });
                 else
-                    run(KR_K_UPDATE, [&] { sweep_hyd<FT>(mp, step, c->variant, (unsigned)c->npure); },
-                        true);
+                    run(KR_K_UPDATE, [&] { sweep_hyd<FT>(mp, step, c->variant, (unsigned)c->npure); });
             }
             ms.blist = c->d_xblk;
             ns = (unsigned)c->nxblk;
         }
         if (ns == 0) return;
-        if (MHD && c->smr && c->prod >= 0) {
+        if (MHD && c->smr && fused && c->prod >= 0) {
             // producer form: fluxes and EMFs into F / EE (the mixed form ran
             // it in the launch above)
             if constexpr (!std::is_same_v<FT, float>)
@@ -1085,7 +1121,7 @@ struct Launcher {
             // shared edges, flux restriction on the faces whose neighbour is
             // finer), then the update with the finer side's EMF write-back and
             // intg_flx folded in
-            const int nx = MHD ? c->nxblk : 0;
+            const int nx = MHD ? c->nxblk : 0;      // blocks whose edges a finer one shares
             if (nx + c->nftask) {
                 // largest face side; one row covers an edge box (MHD) or at
                 // least one face side, tpr face tasks per row

@@ -14,7 +14,7 @@
 //      plane L-2 and z-face L-1.
 // k_sweep is the mixed form's kernel (FP32 fluxes, FP64 state) for meshes
 // with physical sides and refined ones; kr_sweep_mx.h has the one for
-// one-level periodic meshes, kr_sweep64.h the FP64 form's.  PLM is evaluated
+// one-level periodic meshes, kr_march.h the FP64 form's.  PLM is evaluated
 // per cell: the reference's two face states of a cell share one limited
 // increment t, q_l(face i+1) = q_i + t and q_r(face i) = q_i + (-t) exactly
 // (hydro/reconstruct/plm.h:116-153).
@@ -83,15 +83,10 @@ __device__ __forceinline__ float cross_f32(float a, float b, float c, float d) {
 // face EMFs / upwind mass fluxes (mhd/integrator/integrator.h:244-317).
 // ec[s2][s1] naming of the reference: ec11 = E(i), ec10 = E(i - e1),
 // ec00 = E(i - e1 - e2), ec01 = E(i - e2).
-template <class FT>
-__device__ __forceinline__ FT edge_emf(FT ec11, FT ec10, FT ec00, FT ec01, FT efm1, FT efp1,
-                                       FT rp1, FT rm1, FT efm2, FT efp2, FT rp2, FT rm2);
-
-// FP32 (mixed form): the same expression with multiply-add contraction.
-template <>
-__device__ __forceinline__ float edge_emf<float>(float ec11, float ec10, float ec00, float ec01,
-                                                 float efm1, float efp1, float rp1, float rm1,
-                                                 float efm2, float efp2, float rp2, float rm2) {
+// corner_emf with multiply-add contraction (mixed form).
+__device__ __forceinline__ float edge_emf(float ec11, float ec10, float ec00, float ec01, float efm1,
+                                          float efp1, float rp1, float rm1, float efm2, float efp2,
+                                          float rp2, float rm2) {
 #pragma clang fp contract(fast)
     const float w_e = 0.25f;
     float ee = 0;
@@ -105,29 +100,6 @@ __device__ __forceinline__ float edge_emf<float>(float ec11, float ec10, float e
     {
         const float de_p = (rp2 > 0 ? (ec10 - efm2) : (ec11 - efp2));
         const float de_m = (rm2 > 0 ? -(ec00 - efm2) : -(ec01 - efp2));
-        ee += w_e * (de_m - de_p);
-    }
-    return ee;
-}
-
-template <>
-__device__ __forceinline__ double edge_emf<double>(double ec11, double ec10, double ec00,
-                                                   double ec01, double efm1, double efp1,
-                                                   double rp1, double rm1, double efm2,
-                                                   double efp2, double rp2, double rm2) {
-    using FT = double;
-    const FT w_e = (FT)0.25f;
-    FT ee = 0;
-    ee += w_e * (efm1 + efp1);
-    {
-        const FT de_p = (rp1 > 0 ? (ec01 - efm1) : (ec11 - efp1));
-        const FT de_m = (rm1 > 0 ? -(ec00 - efm1) : -(ec10 - efp1));
-        ee += w_e * (de_m - de_p);
-    }
-    ee += w_e * (efm2 + efp2);
-    {
-        const FT de_p = (rp2 > 0 ? (ec10 - efm2) : (ec11 - efp2));
-        const FT de_m = (rm2 > 0 ? -(ec00 - efm2) : -(ec01 - efp2));
         ee += w_e * (de_m - de_p);
     }
     return ee;
@@ -529,7 +501,7 @@ k_sweep(MeshView<float> m, int step) {
                     if (p >= z1) continue;
                     const int x = it % (TX + 1), y = it / (TX + 1);
                     // ee_z on plane p: a1 = x, a2 = y
-                    FT e = edge_emf<FT>(
+                    FT e = edge_emf(
                         ec(s0, x, y, 2), ec(s0, x - 1, y, 2), ec(s0, x - 1, y - 1, 2), ec(s0, x, y - 1, 2),
                         sFez[S::fxi(x, y - 1)], sFez[S::fxi(x, y)],
                         sFe[fe][0][S::fyi(x, y)], sFe[fe][0][S::fyi(x - 1, y)],
@@ -543,7 +515,7 @@ k_sweep(MeshView<float> m, int step) {
                     const int k = it - S::NEZ;
                     const int x = k % TX, y = k / TX;
                     // ee_x on z face p: a1 = y, a2 = z
-                    FT e = edge_emf<FT>(
+                    FT e = edge_emf(
                         ec(s0, x, y, 0), ec(s0, x, y - 1, 0), ec(sm, x, y - 1, 0), ec(sm, x, y, 0),
                         sFe[fm][1][S::fyi(x, y)], sFe[fe][1][S::fyi(x, y)],
                         sFz[0][S::zg(x, y)], sFz[0][S::zg(x, y - 1)],
@@ -557,7 +529,7 @@ k_sweep(MeshView<float> m, int step) {
                     const int k = it - S::NEZ - S::NEX;
                     const int x = k % (TX + 1), y = k / (TX + 1);
                     // ee_y on z face p: a1 = z, a2 = x
-                    FT e = edge_emf<FT>(
+                    FT e = edge_emf(
                         ec(s0, x, y, 1), ec(sm, x, y, 1), ec(sm, x - 1, y, 1), ec(s0, x - 1, y, 1),
                         sFz[2][S::zg(x - 1, y)], sFz[2][S::zg(x, y)],
                         sFe[fe][0][S::fxi(x, y)], sFe[fm][0][S::fxi(x, y)],

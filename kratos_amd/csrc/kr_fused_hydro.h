@@ -39,8 +39,11 @@ __global__ void __launch_bounds__(NT) k_sweep_hyd(MeshView<FT> m, int step) {
     if (m.ts[m.geo[row_block(m)].grp].skip) return;
     const int tid = threadIdx.x;
     const int b = row_block(m);
-    const int ntx = m.n[0] / TX;
-    const int x0 = (blockIdx.x % ntx) * TX, y0 = (blockIdx.x / ntx) * TY;
+    // the last tile along an axis is moved back into the block and leaves the
+    // columns it shares to the one before (kr_march.h)
+    const int ntx = (m.n[0] + TX - 1) / TX;
+    const int xs = (blockIdx.x % ntx) * TX, ys = (blockIdx.x / ntx) * TY;
+    const int x0 = xs + TX > m.n[0] ? m.n[0] - TX : xs, y0 = ys + TY > m.n[1] ? m.n[1] - TY : ys;
     const int nz = m.n[2];
     int z0, z1;
     z_range(nz, z0, z1);
@@ -106,8 +109,8 @@ __global__ void __launch_bounds__(NT) k_sweep_hyd(MeshView<FT> m, int step) {
     };
 
     // owned column of a pencil lane
-    const bool own = tid < OWN;
-    const int cx = own ? tid % TX : 0, cy = own ? tid / TX : 0;
+    const int cx = tid < OWN ? tid % TX : 0, cy = tid < OWN ? tid / TX : 0;
+    const bool own = tid < OWN && cx >= xs - x0 && cy >= ys - y0;
     FT qL[5];                 // left state of the next z face
     FT fzp[5];                // z flux of the previous face
     double part[5];           // x + y partial update of the previous plane

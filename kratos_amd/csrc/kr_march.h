@@ -1,6 +1,8 @@
-// kr_sweep64.h -- fused MHD stage kernel of the FP64 form: the z march, LDS
-// ring, edge EMFs, update and constrained transport of k_sweep (kr_fused.h),
-// with the Riemann solves of a plane spread evenly over the waves.
+// kr_march.h -- fused MHD stage kernel: the z march, LDS ring, edge EMFs,
+// update and constrained transport of k_sweep (kr_fused.h), with the Riemann
+// solves of a plane spread evenly over the waves, for blocks of any size from
+// one tile up.  It runs the FP64 form, and the mixed form (FP32 fluxes, FP64
+// state) on blocks that k_sweep_mx's tiles do not divide.
 //
 // The FP64 solves bound the kernel: a second workgroup on a compute unit
 // gains nothing (time follows the workgroups per compute unit), so what
@@ -13,8 +15,17 @@
 // owned columns' z pencils keep their state in registers (they are the first
 // round's first waves); the columns around, which only feed the EMFs, keep
 // their left state in LDS.  The per-face arithmetic and its order are those
-// of the staged kernels, so the results equal them and the oracle bit for
-// bit.
+// of the staged kernels (kr_exact64.h in FP64), so the results equal theirs,
+// and in FP64 the oracle's, bit for bit.
+//
+// Where the tile does not divide the block, its last tile along an axis is
+// moved back into the block and shares columns with the one before: both
+// compute them, the one before stores them.  The shared columns and the
+// staged kernels' five launches cost about the same where the tiles fill the
+// GPU (300,000 cells in 20x12x25 blocks, mixed: 254 against 256 us a cycle),
+// so the tuner times both there; on fewer cells the march wins (12,000 cells:
+// 95 against 117 us), as on blocks a little larger than its tiles (24^3 in
+// 96^3, FP64: 739 against 903 us).
 #pragma once
 
 #include "kr_exact64.h"
@@ -34,12 +45,15 @@ struct Tile64 {
     __device__ static int iy(int x, int y) { return NIX + y * TX + x; }
 };
 
+// Workgroups along an axis of n cells.
+__host__ __device__ inline int march_tiles(int n, int t) { return (n + t - 1) / t; }
+
 // PROD = 1 (refined meshes, blocks that touch another level): the kernel only
 // produces the fluxes (F) and edge EMFs (EE) of the block, as k_sweep's
 // producer form does.  PHY: meshes with physical sides.
-template <int TX, int TY, int NT, int PROD = 0, bool PHY = false>
-__global__ void __launch_bounds__(NT) k_sweep64(MeshView<double> m, int step) {
-    using FT = double;
+template <class FT, int TX, int TY, int NT, int PROD = 0, bool PHY = false>
+__global__ void __launch_bounds__(NT) k_march(MeshView<FT> m, int step) {
+    constexpr bool F32 = std::is_same_v<FT, float>;
     using S = TileShape<TX, TY>;
     using T = Tile64<TX, TY>;
     constexpr int NROUND = (T::NITEM + NT - 1) / NT;
@@ -48,8 +62,11 @@ __global__ void __launch_bounds__(NT) k_sweep64(MeshView<double> m, int step) {
     if (m.ts[m.geo[row_block(m)].grp].skip) return;
     const int tid = threadIdx.x;
     const int b = row_block(m);
-    const int ntx = m.n[0] / TX;
-    const int x0 = (blockIdx.x % ntx) * TX, y0 = (blockIdx.x / ntx) * TY;
+    const int ntx = march_tiles(m.n[0], TX);
+    const int xs = (blockIdx.x % ntx) * TX, ys = (blockIdx.x / ntx) * TY;
+    // first column and row of the tile, and of its own cells in it
+    const int x0 = xs + TX > m.n[0] ? m.n[0] - TX : xs, y0 = ys + TY > m.n[1] ? m.n[1] - TY : ys;
+    const int ox = xs - x0, oy = ys - y0;
     const int nz = m.n[2];
     int z0, z1;
     z_range(nz, z0, z1);
@@ -59,7 +76,8 @@ __global__ void __launch_bounds__(NT) k_sweep64(MeshView<double> m, int step) {
     const size_t nc = m.ncell;
     const Gam64 gam{m.gamma, m.cv, m.ge};
 
-    constexpr int NDW = S::NCOL * 2;                               // dwords per row
+    constexpr int DPC = (int)sizeof(FT) / 4;                       // dwords per column
+    constexpr int NDW = S::NCOL * DPC;                             // dwords per row
     constexpr int NCHUNK = (NDW + 63) / 64;                        // chunks per row
     __shared__ FT sW[3][8][S::NCOL];
     __shared__ FT sFr[2][S::NF];        // in-plane faces of two planes: mass flux ...
@@ -125,7 +143,7 @@ __global__ void __launch_bounds__(NT) k_sweep64(MeshView<double> m, int step) {
             if ((g.phy >> (2 * a + (da > 0))) & 1) {
                 const int side = da > 0;
                 const int kind = m.bnd[2 * a + side];
-                if (kind == 4) return c == 0 ? m.fix_b[0] : (c == 1 ? m.fix_b[1] : m.fix_b[2]);
+                if (kind == 4) return (FT)(c == 0 ? m.fix_b[0] : (c == 1 ? m.fix_b[1] : m.fix_b[2]));
                 double sgn = 1;
                 const bool top = (g.phy >> (2 * c + 1)) & 1;
 #pragma unroll
@@ -140,7 +158,8 @@ __global__ void __launch_bounds__(NT) k_sweep64(MeshView<double> m, int step) {
                     }
                     if (x == c && top && p[x] >= m.n[x]) p[x] = m.n[x] - 1;
                 }
-                return sgn * m.BF[(((size_t)b * 2 + step) * 3 + c) * m.nface + fidx(m.n, p[0], p[1], p[2])];
+                return (FT)(sgn * m.BF[(((size_t)b * 2 + step) * 3 + c) * m.nface +
+                                       fidx(m.n, p[0], p[1], p[2])]);
             }
         }
         if constexpr (PROD) {
@@ -157,7 +176,7 @@ __global__ void __launch_bounds__(NT) k_sweep64(MeshView<double> m, int step) {
 #pragma unroll
             for (int a = 0; a < 3; ++a) p[a] -= d[a] * m.n[a];
         }
-        return m.BF[(((size_t)blk * 2 + step) * 3 + c) * m.nface + fidx(m.n, p[0], p[1], p[2])];
+        return (FT)m.BF[(((size_t)blk * 2 + step) * 3 + c) * m.nface + fidx(m.n, p[0], p[1], p[2])];
     };
     // asynchronous load of plane z of W into ring slot `slot`
     auto issue_w = [&](int z, int slot) {
@@ -165,20 +184,20 @@ __global__ void __launch_bounds__(NT) k_sweep64(MeshView<double> m, int step) {
         for (int k = wave; k < NCHUNK; k += NT / 64) {
             const int d = k * 64 + lane;
             if (d >= NDW) continue;                 // past the row: no load, no write
-            const int col = d / 2;
-            const int half = d - col * 2;
+            const int col = d / DPC;
+            const int half = d - col * DPC;
             const FT *src = wsrc(col % S::HX - 2, col / S::HX - 2, z);
 #pragma unroll
             for (int v = 0; v < 8; ++v) {
                 const char *gp = (const char *)(src + (size_t)v * nc) + 4 * half;
-                __builtin_amdgcn_global_load_lds(gp, &sW[slot][v][0] + k * 32, 4, 0, 0);
+                __builtin_amdgcn_global_load_lds(gp, &sW[slot][v][0] + k * (64 / DPC), 4, 0, 0);
             }
         }
     };
 
     // owned column of the first NZ threads
-    const bool zint = tid < T::NZ;
-    const int cx_ = zint ? tid % TX : 0, cy_ = zint ? tid / TX : 0;
+    const int cx_ = tid < T::NZ ? tid % TX : 0, cy_ = tid < T::NZ ? tid / TX : 0;
+    const bool zint = tid < T::NZ && cx_ >= ox && cy_ >= oy;
     FT qL[7];                 // left state of the next z face, z frame
     FT fzp[5];                // hydro z flux of the previous face
     double part[5];           // x + y partial update of the previous plane
@@ -192,8 +211,8 @@ __global__ void __launch_bounds__(NT) k_sweep64(MeshView<double> m, int step) {
     // high sides of the block: threads TX*TY .. +TY-1 own the x faces at
     // x = TX, the next TX threads the y faces at y = TY
     const int et = tid - TX * TY;
-    const bool xedge = xlast && et >= 0 && et < TY;
-    const bool yedge = ylast && et >= TY && et < TY + TX;
+    const bool xedge = xlast && et >= oy && et < TY;
+    const bool yedge = ylast && et >= TY + ox && et < TY + TX;
 
     issue_w(z0 - 2, ring3(z0 - 2));
     for (int L = z0 - 2; L <= z1 + 1; ++L) {
@@ -259,7 +278,15 @@ __global__ void __launch_bounds__(NT) k_sweep64(MeshView<double> m, int step) {
                         lo[j] = c[j] - q[sm * PL + v];
                         hi[j] = q[sp * PL + v] - c[j];
                     }
-                    plm_inc64<7>(lo, hi, t);
+                    if constexpr (F32) {
+#pragma unroll
+                        for (int j = 0; j < 7; ++j) {
+                            const int v = vz[j] * S::NCOL;
+                            t[j] = plm_inc_fast(q[sm * PL + v], c[j], q[sp * PL + v]);
+                        }
+                    } else {
+                        plm_inc64<7>(lo, hi, t);
+                    }
 #pragma unroll
                     for (int j = 0; j < 7; ++j) {
                         wl[slot[j]] = qL[j];
@@ -286,12 +313,17 @@ __global__ void __launch_bounds__(NT) k_sweep64(MeshView<double> m, int step) {
                         const FT *q = q0p + off[j];
                         c[j] = q[0];
                         ql[j] = q[om];
-                        lo[j] = c[j] - ql[j];
-                        hi[j] = q[op] - c[j];
-                        lo[7 + j] = ql[j] - q[om2];
-                        hi[7 + j] = lo[j];
+                        if constexpr (F32) {
+                            t[j] = plm_inc_fast(ql[j], c[j], q[op]);
+                            t[7 + j] = plm_inc_fast(q[om2], ql[j], c[j]);
+                        } else {
+                            lo[j] = c[j] - ql[j];
+                            hi[j] = q[op] - c[j];
+                            lo[7 + j] = ql[j] - q[om2];
+                            hi[7 + j] = lo[j];
+                        }
                     }
-                    plm_inc64<14>(lo, hi, t);
+                    if constexpr (!F32) plm_inc64<14>(lo, hi, t);
 #pragma unroll
                     for (int j = 0; j < 7; ++j) {
                         const FT wq = sQ[j][ri];
@@ -303,7 +335,8 @@ __global__ void __launch_bounds__(NT) k_sweep64(MeshView<double> m, int step) {
                 if (a == 2 && p < z0) continue;      // a range's lead-in cell
                 wl[BCC] = bn;
                 wr[BCC] = bn;
-                hlld64(flx, wl, wr, gam);
+                if constexpr (F32) hlld_fast(flx, wl, wr, (FT)m.gamma);
+                else hlld64(flx, wl, wr, gam);
                 if (a == 2) {
                     // rotated frame (z, x, y): E_x = flx[B_y], E_y = -flx[B_x]
                     const int gz = S::zg(fx, fy);
@@ -321,15 +354,15 @@ __global__ void __launch_bounds__(NT) k_sweep64(MeshView<double> m, int step) {
                             }
                         } else {
                             // z part of the cell finished now (plane P)
-                            if (P >= z0) {
-                                const FT fa = sGeo[3 + 2];
+                            if (P >= z0 && zint) {
+                                const FT fa = (FT)sGeo[3 + 2];
                                 double *Ut = m.U + ((size_t)b * 2 + (1 - step)) * 5 * nc +
                                              cidx(m.n, x0 + fx, y0 + fy, P);
 #pragma unroll
                                 for (int v = 0; v < 5; ++v) {
                                     double res(0);
-                                    if (fa > 0) res += fa * fzp[v];
-                                    if (fa > 0) res -= fa * f[v];
+                                    if (fa > 0) res += (double)(fa * fzp[v]);
+                                    if (fa > 0) res -= (double)(fa * f[v]);
                                     Ut[(size_t)v * nc] = part[v] + res;
                                 }
                             }
@@ -417,7 +450,7 @@ __global__ void __launch_bounds__(NT) k_sweep64(MeshView<double> m, int step) {
                     if (p >= z1) continue;
                     const int x = it % (TX + 1), y = it / (TX + 1);
                     // ee_z on plane p: a1 = x, a2 = y
-                    FT e = edge_emf<FT>(
+                    FT e = corner_emf<FT>(
                         ec(s0, x, y, 2), ec(s0, x - 1, y, 2), ec(s0, x - 1, y - 1, 2), ec(s0, x, y - 1, 2),
                         sFez[S::fxi(x, y - 1)], sFez[S::fxi(x, y)], sFr[fe][S::fyi(x, y)],
                         sFr[fe][S::fyi(x - 1, y)], sFez[S::fyi(x - 1, y)], sFez[S::fyi(x, y)],
@@ -430,7 +463,7 @@ __global__ void __launch_bounds__(NT) k_sweep64(MeshView<double> m, int step) {
                     const int k = it - S::NEZ;
                     const int x = k % TX, y = k / TX;
                     // ee_x on z face p: a1 = y, a2 = z
-                    FT e = edge_emf<FT>(
+                    FT e = corner_emf<FT>(
                         ec(s0, x, y, 0), ec(s0, x, y - 1, 0), ec(sm, x, y - 1, 0), ec(sm, x, y, 0),
                         sFt[fm][T::iy(x, y)], sFt[fe][T::iy(x, y)], sFz[0][S::zg(x, y)],
                         sFz[0][S::zg(x, y - 1)], sFz[1][S::zg(x, y - 1)], sFz[1][S::zg(x, y)],
@@ -443,7 +476,7 @@ __global__ void __launch_bounds__(NT) k_sweep64(MeshView<double> m, int step) {
                     const int k = it - S::NEZ - S::NEX;
                     const int x = k % (TX + 1), y = k / (TX + 1);
                     // ee_y on z face p: a1 = z, a2 = x
-                    FT e = edge_emf<FT>(
+                    FT e = corner_emf<FT>(
                         ec(s0, x, y, 1), ec(sm, x, y, 1), ec(sm, x - 1, y, 1), ec(s0, x - 1, y, 1),
                         sFz[2][S::zg(x - 1, y)], sFz[2][S::zg(x, y)], sFr[fe][S::fxi(x, y)],
                         sFr[fm][S::fxi(x, y)], sFt[fm][T::ix(x, y)], sFt[fe][T::ix(x, y)],
@@ -516,14 +549,14 @@ __global__ void __launch_bounds__(NT) k_sweep64(MeshView<double> m, int step) {
                         const int e1 = a == 0 ? S::fxi(x + 1, y) : S::fyi(x, y + 1);
                         const int i0 = a == 0 ? T::ix(x, y) : T::iy(x, y);
                         const int i1 = a == 0 ? T::ix(x + 1, y) : T::iy(x, y + 1);
-                        const double fa = sGeo[3 + a];
+                        const FT fa = (FT)sGeo[3 + a];
 #pragma unroll
                         for (int v = 0; v < 5; ++v) {
                             double res(0);
                             const FT f0 = v == 0 ? sFr[fq][e0] : sFh[v - 1][i0];
                             const FT f1 = v == 0 ? sFr[fq][e1] : sFh[v - 1][i1];
-                            if (fa > 0) res += fa * f0;
-                            if (fa > 0) res -= fa * f1;
+                            if (fa > 0) res += (double)(fa * f0);
+                            if (fa > 0) res -= (double)(fa * f1);
                             uu[v] += res;
                         }
                     }

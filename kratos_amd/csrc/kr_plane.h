@@ -28,29 +28,6 @@
 
 namespace kr {
 
-// Edge EMF of an edge between two active axes (k_emf's expressions, with its
-// rounding also in FP32): cell E at the four corners and the face EMFs and
-// mass fluxes of both directions.
-template <class FT>
-__device__ __forceinline__ FT corner_emf(FT ec11, FT ec10, FT ec00, FT ec01, FT efm1, FT efp1, FT rp1,
-                                         FT rm1, FT efm2, FT efp2, FT rp2, FT rm2) {
-    const FT w_e = (FT)0.25f;
-    FT ee = 0;
-    ee += w_e * (efm1 + efp1);
-    {
-        const FT de_p = (rp1 > 0 ? (ec01 - efm1) : (ec11 - efp1));
-        const FT de_m = (rm1 > 0 ? -(ec00 - efm1) : -(ec10 - efp1));
-        ee += w_e * (de_m - de_p);
-    }
-    ee += w_e * (efm2 + efp2);
-    {
-        const FT de_p = (rp2 > 0 ? (ec10 - efm2) : (ec11 - efp2));
-        const FT de_m = (rm2 > 0 ? -(ec00 - efm2) : -(ec01 - efp2));
-        ee += w_e * (de_m - de_p);
-    }
-    return ee;
-}
-
 template <class FT, bool MHD, int TX, int TY, int NT, bool C2P>
 __global__ void __launch_bounds__(NT) k_plane(MeshView<FT> m, int step) {
     constexpr int NV = MHD ? 8 : 5;

@@ -402,7 +402,7 @@ __global__ void __launch_bounds__(NT, (MODE == MX_LIST && NT <= 256) ? 3 : 1)
                         if (it >= S::NEZ || p >= z1) continue;
                         const int x = it % (TX + 1), y = it / (TX + 1);
                         // ee_z on plane p: a1 = x, a2 = y
-                        sEz[fe][S::ezi(x, y)] = edge_emf<FT>(
+                        sEz[fe][S::ezi(x, y)] = edge_emf(
                             ec(s0, x, y, 2), ec(s0, x - 1, y, 2), ec(s0, x - 1, y - 1, 2), ec(s0, x, y - 1, 2),
                             sFez[S::fxi(x, y - 1)], sFez[S::fxi(x, y)], sFe[fe][0][S::fyi(x, y)],
                             sFe[fe][0][S::fyi(x - 1, y)], sFez[S::fyi(x - 1, y)], sFez[S::fyi(x, y)],
@@ -412,7 +412,7 @@ __global__ void __launch_bounds__(NT, (MODE == MX_LIST && NT <= 256) ? 3 : 1)
                         if (k >= S::NEX) continue;
                         const int x = k % TX, y = k / TX;
                         // ee_x on z face p: a1 = y, a2 = z
-                        sEx[fe][S::exi(x, y)] = edge_emf<FT>(
+                        sEx[fe][S::exi(x, y)] = edge_emf(
                             ec(s0, x, y, 0), ec(s0, x, y - 1, 0), ec(sm, x, y - 1, 0), ec(sm, x, y, 0),
                             sFe[fm][1][S::fyi(x, y)], sFe[fe][1][S::fyi(x, y)], sFz[0][S::zg(x, y)],
                             sFz[0][S::zg(x, y - 1)], sFz[1][S::zg(x, y - 1)], sFz[1][S::zg(x, y)],
@@ -422,7 +422,7 @@ __global__ void __launch_bounds__(NT, (MODE == MX_LIST && NT <= 256) ? 3 : 1)
                         if (k >= S::NEY) continue;
                         const int x = k % (TX + 1), y = k / (TX + 1);
                         // ee_y on z face p: a1 = z, a2 = x
-                        sEy[fe][S::eyi(x, y)] = edge_emf<FT>(
+                        sEy[fe][S::eyi(x, y)] = edge_emf(
                             ec(s0, x, y, 1), ec(sm, x, y, 1), ec(sm, x - 1, y, 1), ec(s0, x - 1, y, 1),
                             sFz[2][S::zg(x - 1, y)], sFz[2][S::zg(x, y)], sFe[fe][0][S::fxi(x, y)],
                             sFe[fm][0][S::fxi(x, y)], sFe[fm][1][S::fxi(x, y)], sFe[fe][1][S::fxi(x, y)],
