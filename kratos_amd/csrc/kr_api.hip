@@ -162,6 +162,10 @@ unsigned z_ranges(size_t wgs, int ncu, int per_cu, int nz, double lat) {
     return best;
 }
 
+// Most resident workgroups of a stage kernel per compute unit (the work list
+// is sized for it; three waves a workgroup and 32 a compute unit allow 10).
+constexpr int kMaxPerCu = 10;
+
 // Doubles of one half of the transfer buffer (1 MiB): while the host copies
 // one half, the GPU fills the other.
 constexpr size_t kPinDoubles = 131072;
@@ -730,13 +734,17 @@ void commit(kr_ctx *c) {
         c->tune_next = 0;
         c->tuned = c->candidates.size() <= 1;
         // an ensemble in the mixed form: k_sweep_mx walks a device work list
-        // of the boxes still running (room for the most tiles, 8x8, in up to
-        // n_z / 8 z-ranges each)
+        // of the boxes still running (room for the most tiles, 8x8, of which
+        // fewer than the resident workgroups are split)
         if (c->fused && mxmesh && c->ngrp > 1) {
             c->mx_list = true;
+            int dev = 0;
+            KR_HIP(hipGetDevice(&dev));
+            KR_HIP(hipDeviceGetAttribute(&c->ncu, hipDeviceAttributeMultiprocessorCount, dev));
             const size_t ntile_max = (size_t)(c->n[0] / 8) * (size_t)(c->n[1] / 8);
-            const size_t kz_max = (size_t)std::max(1, c->n[2] / 8);
-            c->d_items = dalloc<int4>(nb * ntile_max * kz_max);
+            const size_t kz_max = (size_t)std::max(1, c->n[2] / kListRange);
+            const size_t rem_max = std::min(nb * ntile_max, (size_t)c->ncu * kMaxPerCu);
+            c->d_items = dalloc<int4>(nb * ntile_max + rem_max * kz_max);
             c->d_nitems = dalloc<int>(1);
         }
     }
@@ -870,7 +878,7 @@ struct Launcher {
         int &n = c->per_cu[variant];
         if (n == 0) {
             KR_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, fn, threads, 0));
-            n = std::max(1, n);
+            n = std::min(std::max(1, n), kMaxPerCu);
         }
         return n;
     }
@@ -955,9 +963,9 @@ struct Launcher {
         default: march_t<double, 8, 8, 192>(m, step, nb); break;
         }
     }
-    // Ensembles: the stage's work list (the tiles of the boxes still
-    // running, split into more z-ranges as fewer remain), then a persistent
-    // grid of as many workgroups as the GPU holds at once walking it.
+    // Ensembles: the cycle's work list (the tiles of the boxes still running,
+    // split into more z ranges as fewer remain), then a persistent grid of as
+    // many workgroups as the GPU holds at once walking it.
     template <int TX, int TY, int NT>
     void sweep_mx_t(const MeshView<float> &m, int step, unsigned nb) {
         const unsigned nt = (unsigned)((c->n[0] / TX) * (c->n[1] / TY));
@@ -972,10 +980,12 @@ struct Launcher {
         const int per = resident(
             c->variant, reinterpret_cast<const void *>(k_sweep_mx<TX, TY, NT, MX_LIST>), NT);
         const int slots = c->ncu * per;
+        // which boxes run does not change within a cycle
         const unsigned lt = (unsigned)std::min<size_t>(1024, ceil_div((size_t)nb, 64) * 64);
-        hipLaunchKernelGGL(k_sweep_list, dim3(1), dim3(lt), 0, c->stream, (const TimeState *)c->ts,
-                           (const BlockGeo *)c->geo, (int)nb, (int)nt, c->n[2], slots, c->d_items,
-                           c->d_nitems);
+        if (step == 0)
+            hipLaunchKernelGGL(k_sweep_list, dim3(1), dim3(lt), 0, c->stream, (const TimeState *)c->ts,
+                               (const BlockGeo *)c->geo, (int)nb, (int)nt, c->n[2], c->ncu, per,
+                               (float)kLatMhdMixed, c->d_items, c->d_nitems);
         hipLaunchKernelGGL((k_sweep_mx<TX, TY, NT, MX_LIST>), dim3(slots), dim3(NT), 0, c->stream, m,
                            step, (const int4 *)c->d_items, (const int *)c->d_nitems);
     }

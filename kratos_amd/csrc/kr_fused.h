@@ -70,6 +70,21 @@ __device__ __forceinline__ void z_range(int nz, int &z0, int &z1) {
     z1 = ((int)blockIdx.z + 1) * nz / (int)gridDim.z;
 }
 
+// Workgroups go to the 8 XCDs in turn, so neighbouring tiles would read the
+// halo columns they share through 8 different L2 caches.  xcd_order hands
+// each XCD one contiguous run of a launch's n work items instead, xcd_tile
+// one of (block row, tile).  Measured: 128^3 MHD mixed 251 -> 240 us a
+// launch, 256^3 1,659 -> 1,630; FP64 and hydro 1 to 4%.
+__device__ __forceinline__ unsigned xcd_order(unsigned i, unsigned n) {
+    const unsigned x = i & 7, q = n >> 3, r = n & 7;
+    return x * q + (x < r ? x : r) + (i >> 3);
+}
+__device__ __forceinline__ void xcd_tile(unsigned &tile, unsigned &row) {
+    const unsigned w = xcd_order(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
+    row = w / gridDim.x;
+    tile = w - row * gridDim.x;
+}
+
 __device__ __forceinline__ int ring3(int p) { return ((p % 3) + 3) % 3; }
 __device__ __forceinline__ int ring2(int p) { return (p + 4) & 1; }
 

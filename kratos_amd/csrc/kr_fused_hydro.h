@@ -36,13 +36,15 @@ __global__ void __launch_bounds__(NT) k_sweep_hyd(MeshView<FT> m, int step) {
     constexpr int OWNP = (OWN + 63) / 64 * 64;                 // pencil lanes, padded to waves
     constexpr int NFX = (TX + 1) * TY, NFY = TX * (TY + 1), NF = NFX + NFY;
     static_assert(OWN <= NT, "one owned column per lane");
-    if (m.ts[m.geo[row_block(m)].grp].skip) return;
+    unsigned tile, row;
+    xcd_tile(tile, row);
+    const int b = m.blist ? m.blist[row] : (int)row;
+    if (m.ts[m.geo[b].grp].skip) return;
     const int tid = threadIdx.x;
-    const int b = row_block(m);
     // the last tile along an axis is moved back into the block and leaves the
     // columns it shares to the one before (kr_march.h)
     const int ntx = (m.n[0] + TX - 1) / TX;
-    const int xs = (blockIdx.x % ntx) * TX, ys = (blockIdx.x / ntx) * TY;
+    const int xs = (tile % ntx) * TX, ys = (tile / ntx) * TY;
     const int x0 = xs + TX > m.n[0] ? m.n[0] - TX : xs, y0 = ys + TY > m.n[1] ? m.n[1] - TY : ys;
     const int nz = m.n[2];
     int z0, z1;

@@ -59,11 +59,13 @@ __global__ void __launch_bounds__(NT) k_march(MeshView<FT> m, int step) {
     constexpr int NROUND = (T::NITEM + NT - 1) / NT;
     static_assert(T::NZ <= NT && T::NZ % 64 == 0, "owned columns: whole waves of the first round");
     static_assert(TX * TY + TX + TY <= NT, "one owned cell / edge face per thread");
-    if (m.ts[m.geo[row_block(m)].grp].skip) return;
+    unsigned tile, row;
+    xcd_tile(tile, row);
+    const int b = m.blist ? m.blist[row] : (int)row;
+    if (m.ts[m.geo[b].grp].skip) return;
     const int tid = threadIdx.x;
-    const int b = row_block(m);
     const int ntx = march_tiles(m.n[0], TX);
-    const int xs = (blockIdx.x % ntx) * TX, ys = (blockIdx.x / ntx) * TY;
+    const int xs = (tile % ntx) * TX, ys = (tile / ntx) * TY;
     // first column and row of the tile, and of its own cells in it
     const int x0 = xs + TX > m.n[0] ? m.n[0] - TX : xs, y0 = ys + TY > m.n[1] ? m.n[1] - TY : ys;
     const int ox = xs - x0, oy = ys - y0;

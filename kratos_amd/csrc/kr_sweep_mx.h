@@ -47,8 +47,8 @@ enum { MX_GRID = 0, MX_RANGES = 1, MX_LIST = 2 };
 // build of its own, because range bounds known at run time only cost the
 // full march 4% (256^3 in 32^3 blocks: 4.18 against 4.00 ms per cycle).
 // Work-list launch (MX_LIST, ensembles): a persistent grid walks the items
-// (block, tile, z0, z1) that k_sweep_list wrote for the boxes still running, item i on workgroup
-// i mod gridDim.x.  A partial range [z0, z1) repeats the march's lead-in
+// (block, tile, z0, z1) that k_sweep_list wrote for the boxes still running,
+// gridDim.x of them a round.  A partial range [z0, z1) repeats the march's lead-in
 // planes z0 - 2 .. z0 and computes the faces and edges at its ends as the
 // neighbouring range does, through the same code and from the same inputs,
 // and updates only its own cells and faces, so a split changes no result.
@@ -66,7 +66,7 @@ __global__ void __launch_bounds__(NT, (MODE == MX_LIST && NT <= 256) ? 3 : 1)
     static_assert(M::WZ <= NW, "z pencils on the first waves, one pass");
     static_assert(TX * TY + TX + TY <= NT, "one owned cell / edge face per thread");
     static_assert(M::WR <= NW, "one cell-pass item per thread at most");
-    for (int item = (int)blockIdx.x;; item += (int)gridDim.x) {
+    for (int item = LIST ? (int)xcd_order(blockIdx.x, gridDim.x) : 0;; item += (int)gridDim.x) {
         unsigned row, tile;
         int z0, z1;
         if constexpr (LIST) {
@@ -77,8 +77,7 @@ __global__ void __launch_bounds__(NT, (MODE == MX_LIST && NT <= 256) ? 3 : 1)
             z0 = it.z;
             z1 = it.w;
         } else {
-            row = blockIdx.y;
-            tile = blockIdx.x;
+            xcd_tile(tile, row);
             z0 = 0;
             z1 = m.n[2];
             if constexpr (MODE == MX_RANGES) z_range(m.n[2], z0, z1);
@@ -544,17 +543,19 @@ __global__ void __launch_bounds__(NT, (MODE == MX_LIST && NT <= 256) ? 3 : 1)
     }
 }
 
-// Work list of a stage's k_sweep_mx launch: every tile of the blocks whose
-// time group still runs, in block, tile, range order.  With T such tiles
-// and S resident workgroup slots, the first T - T mod S tiles march their
-// whole column and the last T mod S are split into kz z-ranges (at least 8
-// planes each, kz about S / (T mod S)), so that the persistent grid's
-// workgroups, taking items i, i + S, ..., all finish about together (when
-// T < S, every tile is split: more ranges as fewer boxes remain).  One
-// workgroup.
+// Work list of a cycle's k_sweep_mx launches: every tile of the blocks whose
+// time group still runs, in block, tile, range order.  With T such tiles and
+// S = ncu per_cu resident workgroups, the first T - T mod S tiles march their
+// whole column and the last T mod S (when T < S: every tile) are split into
+// kz z ranges, kz from the cost of a launch that z_ranges (kr_api.hip) uses:
+// (n_z / kz + 2) (lat r + k) for k workgroups a compute unit in r rounds.
+// Rounding S / (T mod S) instead left a third of the last round empty (16
+// boxes of 64^3 on 16x8 tiles: 1,024 items on 768 workgroups; now 1,536).
+// One workgroup.
+constexpr int kListRange = 4;          // fewest planes of a range
 __global__ void __launch_bounds__(1024) k_sweep_list(const TimeState *ts, const BlockGeo *geo, int nb,
-                                                     int ntile, int nz, int slots, int4 *items,
-                                                     int *n_items) {
+                                                     int ntile, int nz, int ncu, int per_cu, float lat,
+                                                     int4 *items, int *n_items) {
     __shared__ int part[1024];
     __shared__ int s_kz, s_full;
     const int t = threadIdx.x, nt = blockDim.x;
@@ -571,10 +572,17 @@ __global__ void __launch_bounds__(1024) k_sweep_list(const TimeState *ts, const 
             part[i] = act;
             act += c;
         }
-        const int tiles = act * ntile, rem = tiles % slots;
-        const int kz_max = nz / 8 > 1 ? nz / 8 : 1;
-        int kz = rem ? (slots + rem / 2) / rem : 1;
-        kz = kz < 1 ? 1 : (kz > kz_max ? kz_max : kz);
+        const int slots = ncu * per_cu, tiles = act * ntile, rem = tiles % slots;
+        int kz = 1;
+        float best = 0.f;
+        for (int q = 1; rem && q <= (nz / kListRange > 1 ? nz / kListRange : 1); ++q) {
+            const int k = (rem * q + ncu - 1) / ncu, r = (k + per_cu - 1) / per_cu;
+            const float t = ((float)((nz + q - 1) / q) + 2.f) * (lat * (float)r + (float)k);
+            if (q == 1 || t < best) {
+                best = t;
+                kz = q;
+            }
+        }
         s_kz = kz;
         s_full = tiles - rem;
         *n_items = s_full + rem * kz;
