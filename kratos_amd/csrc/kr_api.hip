@@ -169,6 +169,9 @@ constexpr int kMaxPerCu = 10;
 // Doubles of one half of the transfer buffer (1 MiB): while the host copies
 // one half, the GPU fills the other.
 constexpr size_t kPinDoubles = 131072;
+// Up to here an upload's kernel reads the buffer over the bus: it does so at a
+// tenth of the bus's rate, but saves the copy's latency (8 us).
+constexpr size_t kReadDoubles = 12288;
 
 // Most c2p workgroups of a mesh whose last one takes the dt (FIN): up to
 // there the arrivals cost less than the two launches they replace (32^3: 128
@@ -281,10 +284,12 @@ struct kr_ctx {
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     kr_stats stats{};
     float tune_ms[kNumSweepVariants] = {0};
-    // page-locked host memory that the kernels address: two halves of
-    // kPinDoubles for a transfer, and two snapshots of the time states
-    double *pin = nullptr;
+    // page-locked host memory that the kernels address: two snapshots of the
+    // time states, and two halves of at most kPinDoubles for a transfer
     TimeState *hts = nullptr;
+    double *pin = nullptr;
+    size_t pin_half = 0;
+    double *d_in = nullptr;         // device copy of the halves, for large uploads
     hipEvent_t pin_ev[2] = {nullptr, nullptr};
 
     // the fused kernels run (or, while tuning, the candidate at hand is one)
@@ -328,10 +333,10 @@ void release(kr_ctx *c) {
     void *bufs[] = {c->U,  c->BF, c->W,       c->F[0],  c->F[1],   c->F[2],  c->EE, c->EC,
                     c->geo, c->ts, c->grp_first, c->dt_part, c->red_part, c->red_out,
                     c->d_table, c->d_fill[0], c->d_fill[1], c->d_ftask, c->d_xblk,
-                    c->d_pure, c->d_pfill, c->d_sweep, c->d_items, c->d_nitems, c->arrived};
+                    c->d_pure, c->d_pfill, c->d_sweep, c->d_items, c->d_nitems, c->arrived,
+                    c->d_in};
     for (void *p : bufs)
         if (p) (void)hipFree(p);
-    if (c->pin) (void)hipHostFree(c->pin);
     if (c->hts) (void)hipHostFree(c->hts);
     c->pin = nullptr;
     c->hts = nullptr;
@@ -343,6 +348,7 @@ void release(kr_ctx *c) {
     c->d_items = nullptr;
     c->d_nitems = nullptr;
     c->arrived = nullptr;
+    c->d_in = nullptr;
     c->U = c->BF = nullptr;
     c->W = c->EE = c->EC = nullptr;
     c->F[0] = c->F[1] = c->F[2] = nullptr;
@@ -569,6 +575,22 @@ void build_smr(kr_ctx *c, std::vector<BlockGeo> &g) {
     c->d_sweep = dalloc<int>(rows.size());
     if (!rows.empty())
         KR_HIP(hipMemcpy(c->d_sweep, rows.data(), rows.size() * sizeof(int), hipMemcpyHostToDevice));
+}
+
+HostShape host_shape(const kr_ctx *c, bool bf) {
+    HostShape h{};
+    size_t nf = 1;
+    for (int a = 0; a < 3; ++a) {
+        h.n[a] = c->n[a];
+        // n + (n > 1) faces per axis plus two ghost layers each side
+        // (mhd/types/fld_data.cpp:18-26); a thin axis has one
+        h.N[a] = c->n[a] + (c->n[a] > 1) + 4;
+        nf *= (size_t)h.N[a];
+    }
+    h.nvar = c->mhd ? 8 : 5;
+    h.nu = c->ncell * h.nvar;
+    h.nbf = bf ? nf * 3 : 0;
+    return h;
 }
 
 // Lay out the pools once every block is known (the reference allocates per
@@ -802,8 +824,13 @@ void commit(kr_ctx *c) {
     std::vector<TimeState> tsv(c->ngrp, ts);
     c->ts = dalloc<TimeState>(c->ngrp);
     KR_HIP(hipMemcpy(c->ts, tsv.data(), c->ngrp * sizeof(ts), hipMemcpyHostToDevice));
-    KR_HIP(hipHostMalloc((void **)&c->hts, 2 * c->ngrp * sizeof(TimeState), hipHostMallocDefault));
-    KR_HIP(hipHostMalloc((void **)&c->pin, 2 * kPinDoubles * sizeof(double), hipHostMallocDefault));
+    const HostShape hs = host_shape(c, c->mhd);
+    c->pin_half = std::min(kPinDoubles, hs.nu + hs.nbf);
+    KR_HIP(hipHostMalloc((void **)&c->hts,
+                         2 * c->ngrp * sizeof(TimeState) + 2 * c->pin_half * sizeof(double),
+                         hipHostMallocDefault));
+    c->pin = (double *)(c->hts + 2 * c->ngrp);
+    if (c->pin_half > kReadDoubles) c->d_in = dalloc<double>(2 * c->pin_half);
     c->grp_first = dalloc<int>(c->ngrp + 1);
     KR_HIP(hipMemcpy(c->grp_first, first.data(), (c->ngrp + 1) * sizeof(int), hipMemcpyHostToDevice));
 
@@ -1303,22 +1330,6 @@ double *noalloc_scratch() {
 
 namespace {
 
-HostShape host_shape(const kr_ctx *c, bool bf) {
-    HostShape h{};
-    size_t nf = 1;
-    for (int a = 0; a < 3; ++a) {
-        h.n[a] = c->n[a];
-        // n + (n > 1) faces per axis plus two ghost layers each side
-        // (mhd/types/fld_data.cpp:18-26); a thin axis has one
-        h.N[a] = c->n[a] + (c->n[a] > 1) + 4;
-        nf *= (size_t)h.N[a];
-    }
-    h.nvar = c->mhd ? 8 : 5;
-    h.nu = c->ncell * h.nvar;
-    h.nbf = bf ? nf * 3 : 0;
-    return h;
-}
-
 // [i0, i0 + count) of the host arrays (u, then bf) against one buffer.
 template <class F> void each_part(const HostShape &h, size_t i0, size_t count, F &&f) {
     const size_t i1 = i0 + count;
@@ -1334,20 +1345,20 @@ template <class F> void each_part(const HostShape &h, size_t i0, size_t count, F
 // host work once that kernel has finished.
 template <class Before, class Kernel, class After>
 void transfer(kr_ctx *c, size_t total, Before &&before, Kernel &&kernel, After &&after) {
-    const size_t n = ceil_div(total, kPinDoubles);
+    const size_t half = c->pin_half, n = ceil_div(total, half);
     for (size_t k = 0; k <= n; ++k) {
         if (k < n) {
-            const size_t i0 = k * kPinDoubles, cnt = std::min(kPinDoubles, total - i0);
-            before(i0, cnt, c->pin + (k & 1) * kPinDoubles);
-            kernel(i0, cnt, c->pin + (k & 1) * kPinDoubles);
+            const size_t i0 = k * half, cnt = std::min(half, total - i0);
+            before(i0, cnt, c->pin + (k & 1) * half);
+            kernel(i0, cnt, c->pin + (k & 1) * half);
             KR_HIP(hipGetLastError());
             if (n > 1) KR_HIP(hipEventRecord(c->pin_ev[k & 1], c->stream));
         }
         if (k > 0) {
-            const size_t i0 = (k - 1) * kPinDoubles, cnt = std::min(kPinDoubles, total - i0);
+            const size_t i0 = (k - 1) * half, cnt = std::min(half, total - i0);
             if (n > 1) KR_HIP(hipEventSynchronize(c->pin_ev[(k - 1) & 1]));
             else KR_HIP(hipStreamSynchronize(c->stream));
-            after(i0, cnt, c->pin + ((k - 1) & 1) * kPinDoubles);
+            after(i0, cnt, c->pin + ((k - 1) & 1) * half);
         }
     }
 }
@@ -1366,8 +1377,13 @@ void upload_one(kr_ctx *c, size_t b, const double *u_aos, const double *bf_aos) 
             });
         },
         [&](size_t i0, size_t cnt, const double *buf) {
+            const double *in = buf;
+            if (cnt > kReadDoubles) {
+                in = c->d_in + (buf - c->pin);
+                KR_HIP(hipMemcpyAsync((void *)in, buf, cnt * sizeof(double), hipMemcpyHostToDevice, c->stream));
+            }
             hipLaunchKernelGGL(k_unpack, dim3(ceil_div(cnt, kThreads)), dim3(kThreads), 0, c->stream, h, U,
-                               BF, c->ncell, c->nface, i0, cnt, buf);
+                               BF, c->ncell, c->nface, i0, cnt, in);
         },
         [](size_t, size_t, const double *) {});
 }
