@@ -173,10 +173,13 @@ constexpr size_t kPinDoubles = 131072;
 // tenth of the bus's rate, but saves the copy's latency (8 us).
 constexpr size_t kReadDoubles = 12288;
 
-// Most c2p workgroups of a mesh whose last one takes the dt (FIN): up to
-// there the arrivals cost less than the two launches they replace (32^3: 128
-// workgroups, 92 -> 85 us a cycle).
-constexpr size_t kFinWorkgroups = 1024;
+// Most c2p workgroups of a mesh whose last one takes the dt (FIN): the two
+// launches it replaces cost the same on every mesh, its arrivals add up with
+// the workgroups.  A cycle with the launches and with FIN, mixed MHD: 128
+// workgroups 66.1 and 62.4 us, 288 88.6 and 86.6, 432 89.8 and 90.6, 768 107.9
+// and 112.9, 1,024 124.1 and 137.9; FP64 hydro: 54.1 and 51.4, 71.6 and 70.2,
+// 74.9 and 76.0, 89.6 and 97.6, 112.2 and 124.3.
+constexpr size_t kFinWorkgroups = 320;
 
 // graph replays between host checks of the stop rule in kr_advance
 constexpr int kAdvanceChunk = 64;
