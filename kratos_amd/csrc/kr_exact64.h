@@ -1,6 +1,7 @@
-// kr_exact64.h -- the FP64 flux functions of the fused kernels: the same
-// values as the general ones (plm, hlld and hllc of kr_physics.h) bit for bit, the sign of a zero
-// aside, in fewer instructions and without branches.
+// kr_exact64.h -- the FP64 flux functions of the GPU kernels: the
+// values of the reference's PLM and of the general hlld and hllc of
+// kr_physics.h bit for bit, the sign of a zero aside, in fewer instructions
+// and without branches.
 //
 // What bounds them is the number of FP64 instructions a wave issues; half of
 // hlld<double> is IEEE divisions (31 of about 16 issue slots each, counting
@@ -291,6 +292,34 @@ __device__ __forceinline__ void hllc64(double *flx, const double *wl, const doub
     flx[MOM + 2] = s * (rho * sel(left, wl[MOM + 2], wr[MOM + 2]) * vn);
     flx[MOM] += sm * cp;
     flx[ENE] += sm * cp * am;
+}
+
+// Face flux in the mesh frame for a sweep along `axis`: hllc.h:32-43 and
+// hlld.h:29-47 (the B-flux slots are rewritten as edge EMFs, normal slot 0).
+// ql / qr are rotated in place.
+template <class FT, bool MHD, int AXIS>
+__device__ __forceinline__ void face_flux(FT *ql, FT *qr, FT *flx, const Gam64 &k) {
+    rot<AXIS>(ql + MOM);
+    rot<AXIS>(qr + MOM);
+    if constexpr (MHD) {
+        rot<AXIS>(ql + BCC);
+        rot<AXIS>(qr + BCC);
+        if constexpr (std::is_same_v<FT, float>)
+            hlld_fast(flx, ql, qr, (float)k.g);
+        else
+            hlld64(flx, ql, qr, k);
+        rot<3 - AXIS>(flx + MOM);
+        const FT e0 = flx[BCC + 2], e1 = -flx[BCC + 1];
+        flx[BCC + (AXIS + 1) % 3] = e0;
+        flx[BCC + (AXIS + 2) % 3] = e1;
+        flx[BCC + AXIS] = 0;
+    } else {
+        if constexpr (std::is_same_v<FT, float>)
+            hllc_fast(flx, ql, qr, (float)k.g);
+        else
+            hllc64(flx, ql, qr, k);
+        rot<3 - AXIS>(flx + MOM);
+    }
 }
 
 }  // namespace kr

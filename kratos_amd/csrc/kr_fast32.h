@@ -29,7 +29,7 @@ __device__ __forceinline__ float plm_inc_fast(float qm, float q0, float qp) {
 }
 
 // Face states of the face between cells l and r from the four cells
-// ll, l, r, rr (the per-face form of plm<float>).
+// ll, l, r, rr.
 __device__ __forceinline__ void plm_fast(float q_ll, float q_l, float q_r, float q_rr, float &ql,
                                          float &qr) {
 #pragma clang fp contract(fast)

@@ -148,34 +148,6 @@ __device__ __forceinline__ double dt_mhd_mixed(const double *v_p, const double *
 }
 
 // ---------------------------------------------------------------------
-// PLM on a uniform mesh.  hydro/reconstruct/plm.h:116-153.  The FP32 form
-// rescales the slopes by their largest magnitude (:128-137) to keep the
-// products in range; the FP64 form uses norm = 1.
-template <class FT>
-__device__ __forceinline__ void plm(FT q_ll, FT q_l, FT q_r, FT q_rr, FT &ql, FT &qr) {
-    const FT dql = (q_l - q_ll);
-    const FT dqc = (q_r - q_l);
-    const FT dqr = (q_rr - q_r);
-    FT norm(1);
-    if constexpr (std::is_same_v<FT, float>) {
-        const FT fmin_c = (FT)1e-24f;   // type::float_min at PRECISION 0/1
-        if (kfabs(dqc) > fmin_c || kfabs(dqr) > fmin_c || kfabs(dql) > fmin_c) {
-            norm = pmax(kfabs(dqr), kfabs(dql));
-            norm = 1 / pmax(kfabs(dqc), norm);
-        }
-    }
-    const FT dqr2 = norm * dqr * dqr;
-    const FT dql2 = norm * dql * dql;
-    const FT dqc2 = norm * dqc * dqc;
-    const FT dq2_l = norm * dql * dqc;
-    const FT dq2_r = norm * dqr * dqc;
-    const FT ql_coef = dq2_l <= 0 ? (FT)0 : dq2_l / (dql2 + dqc2 + dq2_l * 2);
-    const FT qr_coef = dq2_r <= 0 ? (FT)0 : -dq2_r / (dqr2 + dqc2 + dq2_r * 2);
-    ql = q_l + (dq2_l <= 0 ? (FT)0 : ql_coef * (dql + dqc));
-    qr = q_r + (dq2_r <= 0 ? (FT)0 : qr_coef * (dqc + dqr));
-}
-
-// ---------------------------------------------------------------------
 // et_cs (hydro/eos/adiabatic.h:62-76) in the flux precision.
 template <class FT>
 __device__ __forceinline__ FT et_cs(FT &e_tot, FT &c_s, const FT *w, FT gam) {
@@ -433,9 +405,6 @@ __device__ __forceinline__ void hlld(FT *flx, const FT *wli, const FT *wri, FT g
 
 namespace kr {
 
-// Face flux in the mesh frame for a sweep along `axis`: hllc.h:32-43 and
-// hlld.h:29-47 (the B-flux slots are rewritten as edge EMFs, normal slot 0).
-// ql / qr are rotated in place.
 // Rotation with a compile-time axis, so that every register array index is
 // static (no scratch spills).
 template <int AXIS, class T> __device__ __forceinline__ void rot(T *x) {
@@ -444,31 +413,6 @@ template <int AXIS, class T> __device__ __forceinline__ void rot(T *x) {
         x[0] = s0;
         x[1] = s1;
         x[2] = s2;
-    }
-}
-
-template <class FT, bool MHD, int AXIS>
-__device__ __forceinline__ void face_flux(FT *ql, FT *qr, FT *flx, FT gam) {
-    rot<AXIS>(ql + MOM);
-    rot<AXIS>(qr + MOM);
-    if constexpr (MHD) {
-        rot<AXIS>(ql + BCC);
-        rot<AXIS>(qr + BCC);
-        if constexpr (std::is_same_v<FT, float>)
-            hlld_fast(flx, ql, qr, gam);
-        else
-            hlld<FT>(flx, ql, qr, gam);
-        rot<3 - AXIS>(flx + MOM);
-        const FT e0 = flx[BCC + 2], e1 = -flx[BCC + 1];
-        flx[BCC + (AXIS + 1) % 3] = e0;
-        flx[BCC + (AXIS + 2) % 3] = e1;
-        flx[BCC + AXIS] = 0;
-    } else {
-        if constexpr (std::is_same_v<FT, float>)
-            hllc_fast(flx, ql, qr, gam);
-        else
-            hllc<FT>(flx, ql, qr, gam);
-        rot<3 - AXIS>(flx + MOM);
     }
 }
 

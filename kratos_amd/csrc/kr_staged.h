@@ -9,7 +9,7 @@
 #pragma once
 
 #include "kr_mesh.h"
-#include "kr_physics.h"
+#include "kr_exact64.h"
 
 namespace kr {
 
@@ -418,6 +418,11 @@ __global__ void __launch_bounds__(kThreads) k_c2p(MeshView<FT> m, int step, cons
 // :334-352 (hydro) or mhd/integrator/data.h:53-141 (MHD lines, including the
 // transverse ghost lines) for the pencil, PLM per face
 // (hydro/reconstruct/plm.h:116-153, mhd/reconstruct/plm.h:18-50).
+//
+// FP64 takes the functions of kr_exact64.h.  Fewer instructions helped little
+// here: the three sweeps over 442 MHD blocks of 8^3 went from 36.6, 36.4 and
+// 34.9 us to 35.2, 34.8 and 32.3 (seven waves a SIMD, of which 148 registers
+// let three run at a time).
 template <class FT, bool MHD, int AXIS>
 __global__ void __launch_bounds__(kThreads) k_flux(MeshView<FT> m, int step) {
     constexpr int axis = AXIS;
@@ -456,20 +461,34 @@ __global__ void __launch_bounds__(kThreads) k_flux(MeshView<FT> m, int step) {
         load_cell<FT, NV>(m, b, pc, q[s]);
     }
     FT ql[NV], qr[NV], flx[NV];
+    if constexpr (std::is_same_v<FT, float>) {
 #pragma unroll
-    for (int v = 0; v < NV; ++v) {
-        if (MHD && v == BCC + axis) continue;
-        if constexpr (std::is_same_v<FT, float>)
+        for (int v = 0; v < NV; ++v) {
+            if (MHD && v == BCC + axis) continue;
             plm_fast(q[0][v], q[1][v], q[2][v], q[3][v], ql[v], qr[v]);
-        else
-            plm<FT>(q[0][v], q[1][v], q[2][v], q[3][v], ql[v], qr[v]);
+        }
+    } else {
+        FT lo[2 * NV], hi[2 * NV], t[2 * NV];
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            const bool bn = MHD && v == BCC + axis;      // taken from the face below
+            lo[v] = bn ? 0 : q[1][v] - q[0][v];
+            hi[v] = lo[NV + v] = bn ? 0 : q[2][v] - q[1][v];
+            hi[NV + v] = bn ? 0 : q[3][v] - q[2][v];
+        }
+        plm_inc64<2 * NV>(lo, hi, t);
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            ql[v] = q[1][v] + t[v];
+            qr[v] = q[2][v] - t[NV + v];
+        }
     }
     if constexpr (MHD) {
         const FT bn = (FT)load_bf(m, b, step, axis, p);
         ql[BCC + axis] = bn;
         qr[BCC + axis] = bn;
     }
-    face_flux<FT, MHD, AXIS>(ql, qr, flx, (FT)m.gamma);
+    face_flux<FT, MHD, AXIS>(ql, qr, flx, Gam64{m.gamma, m.cv, m.ge});
     FT *F = m.F[axis] + (size_t)b * NV * m.nfa[axis] + t;
 #pragma unroll
     for (int v = 0; v < NV; ++v) F[(size_t)v * m.nfa[axis]] = flx[v];
