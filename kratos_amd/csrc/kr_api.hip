@@ -1152,7 +1152,7 @@ struct Launcher {
         });
         if constexpr (MHD)
             run(KR_K_EMF, [&] {
-                hipLaunchKernelGGL(k_emf<FT>, dim3(ceil_div(c->nface, kThreads), ns), blk, 0,
+                hipLaunchKernelGGL(k_emf<FT>, dim3(ceil_div(c->nface, kThreads), ns, 3), blk, 0,
                                    c->stream, ms);
             });
         }

@@ -546,71 +546,81 @@ __device__ __forceinline__ FT flux_at(const MeshView<FT> &m, int b, int a, const
 // come last (m.ndim counts the active ones): they carry one edge layer, no
 // shift, no flux and no corner upwinding, and an edge next to one takes the
 // surviving sweep at weight 0.5 (:221-300).
+template <class FT, int AX>
+__device__ __forceinline__ FT edge_at(const MeshView<FT> &m, int b, int *i) {
+    constexpr int ax = AX, ax_1 = (AX + 1) % 3, ax_2 = (AX + 2) % 3;
+    const int n_dm = m.ndim;
+    const bool th_1 = ax_1 >= n_dm, th_2 = ax_2 >= n_dm;
+    const int axis[3] = {ax, ax_1, ax_2};
+    FT ec[2][2];
+    ec[1][1] = ec_at(m, b, i, axis);
+    if (!th_1) --i[ax_1];
+    ec[1][0] = ec_at(m, b, i, axis);
+    if (!th_2) --i[ax_2];
+    ec[0][0] = ec_at(m, b, i, axis);
+    if (!th_1) ++i[ax_1];
+    ec[0][1] = ec_at(m, b, i, axis);
+    if (!th_2) ++i[ax_2];
+    FT ee = 0;
+    const FT w_e = (th_1 || th_2) ? (FT)0.5f : (FT)0.25f;
+#pragma unroll
+    for (int pi = 0; pi < 2; ++pi) {
+        const int a_para = pi == 0 ? ax_1 : ax_2;
+        const int a_perp = pi == 0 ? ax_2 : ax_1;
+        const bool thn_p = a_perp >= n_dm;
+        if (a_para < n_dm) {
+            if (!thn_p) --i[a_perp];
+            const FT ef_m = flux_at(m, b, a_para, i, BCC + ax);
+            if (!thn_p) ++i[a_perp];
+            const FT ef_p = flux_at(m, b, a_para, i, BCC + ax);
+            ee += w_e * (ef_m + ef_p);
+            if (!thn_p) {
+                const FT frho_p = flux_at(m, b, a_perp, i, RHO);
+                --i[a_para];
+                const FT frho_m = flux_at(m, b, a_perp, i, RHO);
+                ++i[a_para];
+                const FT de_p = (frho_p > 0 ? (ec[0][1] - ef_m) : (ec[1][1] - ef_p));
+                const FT de_m = (frho_m > 0 ? -(ec[0][0] - ef_m) : -(ec[1][0] - ef_p));
+                ee += w_e * (de_m - de_p);
+            }
+        }
+        if (pi == 0) {
+            const FT swp = ec[0][1];
+            ec[0][1] = ec[1][0];
+            ec[1][0] = swp;
+        }
+    }
+    return ee;
+}
+
+// One grid layer (z) per edge direction: an edge waits for its cells, then
+// for its fluxes, behind the branches that find them, and a thread that took
+// its three edges one after another did so three times in a row (442 FP64
+// blocks of 8^3: 38.2 us, with layers 28.3; a cycle of the staged mixed form
+// at 32^3 122.5 and 104.0 us, at 128^3 1,010 and 953).
 template <class FT>
 __global__ void __launch_bounds__(kThreads) k_emf(MeshView<FT> m) {
     if (m.ts[m.geo[row_block(m)].grp].skip) return;
-    const int b = row_block(m);
+    const int b = row_block(m), ax = blockIdx.z;
     const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= m.nface) return;
     int i[3];
     i[0] = (int)(t % (m.n[0] + 1));
     i[1] = (int)((t / (m.n[0] + 1)) % (m.n[1] + 1));
     i[2] = (int)(t / ((size_t)(m.n[0] + 1) * (m.n[1] + 1)));
-    const int n_dm = m.ndim;
-    for (int a = n_dm; a < 3; ++a)
+    for (int a = m.ndim; a < 3; ++a)
         if (i[a] > 0) return;
-    for (int ax = 0; ax < 3; ++ax) {
-        if (i[ax] >= m.n[ax]) continue;
-        const int ax_1 = mod3(1 + ax), ax_2 = mod3(2 + ax);
-        const bool th_1 = ax_1 >= n_dm, th_2 = ax_2 >= n_dm;
-        const int axis[3] = {ax, ax_1, ax_2};
-        FT ec[2][2];
-        ec[1][1] = ec_at(m, b, i, axis);
-        if (!th_1) --i[ax_1];
-        ec[1][0] = ec_at(m, b, i, axis);
-        if (!th_2) --i[ax_2];
-        ec[0][0] = ec_at(m, b, i, axis);
-        if (!th_1) ++i[ax_1];
-        ec[0][1] = ec_at(m, b, i, axis);
-        if (!th_2) ++i[ax_2];
-        FT ee = 0;
-        const FT w_e = (th_1 || th_2) ? (FT)0.5f : (FT)0.25f;
-#pragma unroll
-        for (int pi = 0; pi < 2; ++pi) {
-            const int a_para = pi == 0 ? ax_1 : ax_2;
-            const int a_perp = pi == 0 ? ax_2 : ax_1;
-            const bool thn_p = a_perp >= n_dm;
-            if (a_para < n_dm) {
-                if (!thn_p) --i[a_perp];
-                const FT ef_m = flux_at(m, b, a_para, i, BCC + ax);
-                if (!thn_p) ++i[a_perp];
-                const FT ef_p = flux_at(m, b, a_para, i, BCC + ax);
-                ee += w_e * (ef_m + ef_p);
-                if (!thn_p) {
-                    const FT frho_p = flux_at(m, b, a_perp, i, RHO);
-                    --i[a_para];
-                    const FT frho_m = flux_at(m, b, a_perp, i, RHO);
-                    ++i[a_para];
-                    const FT de_p = (frho_p > 0 ? (ec[0][1] - ef_m) : (ec[1][1] - ef_p));
-                    const FT de_m = (frho_m > 0 ? -(ec[0][0] - ef_m) : -(ec[1][0] - ef_p));
-                    ee += w_e * (de_m - de_p);
-                }
-            }
-            if (pi == 0) {
-                const FT swp = ec[0][1];
-                ec[0][1] = ec[1][0];
-                ec[1][0] = swp;
-            }
-        }
-        m.EE[((size_t)b * 3 + ax) * m.nface + t] = ee;
-    }
+    FT *EE = m.EE + ((size_t)b * 3 + ax) * m.nface + t;
+    if (ax == 0 && i[0] < m.n[0]) *EE = edge_at<FT, 0>(m, b, i);
+    if (ax == 1 && i[1] < m.n[1]) *EE = edge_at<FT, 1>(m, b, i);
+    if (ax == 2 && i[2] < m.n[2]) *EE = edge_at<FT, 2>(m, b, i);
     // boundary-plane advective edge EMF of a high out / fre side
     // (mhd/integrator/integrator.h:328-381): the interior cell's value with
     // v = w[mom] / rho as written there; later axes overwrite earlier ones
     const BlockGeo &g = m.geo[b];
     if (g.phy)
         for (int a = 0; a < 3; ++a) {
-            if (i[a] != m.n[a] || m.n[a] < 2 || !((g.phy >> (2 * a + 1)) & 1)) continue;
+            if (a == ax || i[a] != m.n[a] || m.n[a] < 2 || !((g.phy >> (2 * a + 1)) & 1)) continue;
             const int k = m.bnd[2 * a + 1];
             if (k != 1 && k != 2) continue;
             int jc[3] = {i[0], i[1], i[2]};
@@ -625,8 +635,7 @@ __global__ void __launch_bounds__(kThreads) k_emf(MeshView<FT> m) {
                 b_c[q] = w[BCC + q];
             }
             const int a1 = mod3(a + 1), a2 = mod3(a + 2);
-            m.EE[((size_t)b * 3 + a1) * m.nface + t] = v_c[a] * b_c[a2] - v_c[a2] * b_c[a];
-            m.EE[((size_t)b * 3 + a2) * m.nface + t] = v_c[a1] * b_c[a] - v_c[a] * b_c[a1];
+            *EE = ax == a1 ? v_c[a] * b_c[a2] - v_c[a2] * b_c[a] : v_c[a1] * b_c[a] - v_c[a] * b_c[a1];
         }
 }
 
