@@ -181,6 +181,15 @@ constexpr size_t kReadDoubles = 12288;
 // 74.9 and 76.0, 89.6 and 97.6, 112.2 and 124.3.
 constexpr size_t kFinWorkgroups = 320;
 
+// Most workgroups of a staged MHD update whose cells and three face families
+// are layers of the grid: above, one layer fills the GPU and a point's cell
+// and faces share cache lines.  Four (mixed) and eight (FP64, whose registers
+// hold fewer waves) a compute unit.  A staged cycle with one layer and with
+// four, mixed: 160 workgroups 93.9 and 87.5 us, 3,968 494.2 and 505.4, 8,840
+// 1,347 and 1,387 (even at about 1,350); FP64: 160 117.6 and 113.5, 1,326
+// 449.6 and 443.5, 3,968 810.2 and 813.4, 8,840 2,180 and 2,222.
+template <class FT> constexpr size_t kLayerWorkgroups = std::is_same_v<FT, double> ? 2048 : 1024;
+
 // graph replays between host checks of the stop rule in kr_advance
 constexpr int kAdvanceChunk = 64;
 
@@ -1156,6 +1165,9 @@ struct Launcher {
                                    c->stream, ms);
             });
         }
+        // the update's cells and faces: layers of the grid up to kLayerWorkgroups
+        const unsigned uw = (unsigned)ceil_div(MHD ? c->nface : c->ncell, kThreads);
+        const unsigned ul = MHD && (size_t)uw * ns <= kLayerWorkgroups<FT> ? 4 : 1;
         if (c->smr) {
             // act_flx in one launch (EMF restriction on the coarser blocks'
             // shared edges, flux restriction on the faces whose neighbour is
@@ -1180,14 +1192,14 @@ struct Launcher {
             }
             run(KR_K_UPDATE, [&] {
                 hipLaunchKernelGGL((k_smr_update<FT, MHD>),
-                                   dim3(ceil_div(MHD ? c->nface : c->ncell, kThreads), ns), blk, 0,
+                                   dim3(uw, ns, ul), blk, 0,
                                    c->stream, ms, step);
             });
             return;
         }
         run(KR_K_UPDATE, [&] {
             hipLaunchKernelGGL((k_update<FT, MHD>),
-                               dim3(ceil_div(MHD ? c->nface : c->ncell, kThreads), ns), blk, 0,
+                               dim3(uw, ns, ul), blk, 0,
                                c->stream, ms, step);
         });
     }

@@ -661,7 +661,9 @@ __device__ __forceinline__ void update_point(const MeshView<FT> &m, int b, size_
     i[2] = (int)(t / ((size_t)e0 * e1));
     const double dt = m.ts[m.geo[b].grp].dt_use * (step == 0 ? 1.0 : 0.5);
     const BlockGeo &g = m.geo[b];
-    if (i[0] < m.n[0] && i[1] < m.n[1] && i[2] < m.n[2]) {
+    // grid layer: -1 all of the point, else 0 its cell, 1 + a its face along a
+    const int part = MHD && gridDim.z > 1 ? (int)blockIdx.z : -1;
+    if (part <= 0 && i[0] < m.n[0] && i[1] < m.n[1] && i[2] < m.n[2]) {
         const size_t c = cidx(m.n, i[0], i[1], i[2]);
         const double *Us = m.U + ((size_t)b * 2 + step) * 5 * m.ncell + c;
         double *Ut = m.U + ((size_t)b * 2 + (1 - step)) * 5 * m.ncell + c;
@@ -675,35 +677,39 @@ __device__ __forceinline__ void update_point(const MeshView<FT> &m, int b, size_
                 uu[v] = (Us[(size_t)v * m.ncell] + Ut[(size_t)v * m.ncell]) * 0.5f;
         }
         const double dt_dv = dt / g.vol;
-        for (int ax = 0; ax < m.ndim; ++ax) {
+        // All face fluxes are loaded before the first is used, also those of
+        // faces that the sums below leave out (they lie in the flux box): a
+        // cell waits for memory once and not once behind each condition
+        // (k_smr_update, mixed, 442 blocks of 16^3: 142 -> 113 us).
+        FT f0[3][5], f1[3][5];
+#pragma unroll
+        for (int ax = 0; ax < 3; ++ax) {
+            if (ax >= m.ndim) continue;
             int p1[3] = {i[0], i[1], i[2]};
             ++p1[ax];
             const size_t x0 = xidx(m.n, ax, i), x1 = xidx(m.n, ax, p1);
             const FT *F = m.F[ax] + (size_t)b * NV * m.nfa[ax];
+#pragma unroll
+            for (int v = 0; v < 5; ++v) {
+                f0[ax][v] = F[(size_t)v * m.nfa[ax] + x0];
+                f1[ax][v] = F[(size_t)v * m.nfa[ax] + x1];
+            }
+        }
+#pragma unroll
+        for (int ax = 0; ax < 3; ++ax) {
+            if (ax >= m.ndim) continue;
             // faces whose neighbour is finer are skipped here and added with
             // the restricted flux afterwards (integrator.h:156-182 null_l/r)
             const bool n0 = ((g.rface >> (2 * ax)) & 1) && i[ax] == 0;
             const bool n1 = ((g.rface >> (2 * ax + 1)) & 1) && i[ax] + 1 == m.n[ax];
-            if constexpr (std::is_same_v<FT, double>) {
-                const double fa = g.sfc[ax] * dt_dv;
-                const double fa0 = n0 ? -1 : fa, fa1 = n1 ? -1 : fa;
+            const FT fa = (FT)(g.sfc[ax] * dt_dv);
+            const bool u0 = !n0 && fa > 0, u1 = !n1 && fa > 0;
 #pragma unroll
-                for (int v = 0; v < 5; ++v) {
-                    double res(0);
-                    if (fa0 > 0) res += fa0 * F[(size_t)v * m.nfa[ax] + x0];
-                    if (fa1 > 0) res -= fa1 * F[(size_t)v * m.nfa[ax] + x1];
-                    uu[v] += res;
-                }
-            } else {
-                const float fa = (float)(g.sfc[ax] * dt_dv);
-                const float fa0 = n0 ? -1.f : fa, fa1 = n1 ? -1.f : fa;
-#pragma unroll
-                for (int v = 0; v < 5; ++v) {
-                    double res(0);
-                    if (fa0 > 0) res += (double)(fa0 * F[(size_t)v * m.nfa[ax] + x0]);
-                    if (fa1 > 0) res -= (double)(fa1 * F[(size_t)v * m.nfa[ax] + x1]);
-                    uu[v] += res;
-                }
+            for (int v = 0; v < 5; ++v) {
+                double res(0);
+                res = u0 ? res + (double)(fa * f0[ax][v]) : res;
+                res = u1 ? res - (double)(fa * f1[ax][v]) : res;
+                uu[v] += res;
             }
         }
         finish(i, uu);
@@ -722,7 +728,7 @@ __device__ __forceinline__ void update_point(const MeshView<FT> &m, int b, size_
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
             const int ax_1 = mod3(a + 1), ax_2 = mod3(a + 2);
-            if (i[ax_1] >= m.n[ax_1] || i[ax_2] >= m.n[ax_2]) continue;
+            if ((part >= 0 && part != a + 1) || i[ax_1] >= m.n[ax_1] || i[ax_2] >= m.n[ax_2]) continue;
             // an edge pair spanning a thin axis vanishes
             // (mhd/integrator/integrator.h:419-447)
             const bool th_1 = ax_1 >= m.ndim, th_2 = ax_2 >= m.ndim;
