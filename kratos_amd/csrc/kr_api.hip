@@ -287,6 +287,8 @@ struct kr_ctx {
     int nftask = 0;
     int *d_xblk = nullptr;          // blocks with cross-level sides
     int nxblk = 0;
+    int *d_eblk = nullptr;          // those of them that touch a finer level
+    int neblk = 0;
     int *d_pure = nullptr;          // blocks with no cross-level direction (fused kernel)
     int npure = 0;
     int *d_sweep = nullptr;         // the pure blocks, then the cross-level ones: the rows
@@ -344,7 +346,7 @@ void release(kr_ctx *c) {
     c->graph = nullptr;
     void *bufs[] = {c->U,  c->BF, c->W,       c->F[0],  c->F[1],   c->F[2],  c->EE, c->EC,
                     c->geo, c->ts, c->grp_first, c->dt_part, c->red_part, c->red_out,
-                    c->d_table, c->d_fill[0], c->d_fill[1], c->d_ftask, c->d_xblk,
+                    c->d_table, c->d_fill[0], c->d_fill[1], c->d_ftask, c->d_xblk, c->d_eblk,
                     c->d_pure, c->d_pfill, c->d_sweep, c->d_items, c->d_nitems, c->arrived,
                     c->d_in};
     for (void *p : bufs)
@@ -356,7 +358,7 @@ void release(kr_ctx *c) {
     c->d_fill[0] = c->d_fill[1] = nullptr;
     c->d_pfill = nullptr;
     c->d_ftask = nullptr;
-    c->d_xblk = c->d_pure = c->d_sweep = nullptr;
+    c->d_xblk = c->d_eblk = c->d_pure = c->d_sweep = nullptr;
     c->d_items = nullptr;
     c->d_nitems = nullptr;
     c->arrived = nullptr;
@@ -448,7 +450,7 @@ void build_smr(kr_ctx *c, std::vector<BlockGeo> &g) {
     }
     std::vector<int4> fill[2];
     std::vector<int2> ftask;
-    std::vector<int> xblk, pure;
+    std::vector<int> xblk, eblk, pure;
     int nhalo = 0;
     for (size_t b = 0; b < nb; ++b) {
         const kr_block_desc &d = c->descs[b];
@@ -511,6 +513,7 @@ void build_smr(kr_ctx *c, std::vector<BlockGeo> &g) {
                 }
         bool any = false;
         for (int k = 0; k < 27; ++k) any |= G.lev[k] == 1 || G.lev[k] == -1;
+        if (std::find(G.lev, G.lev + 27, (signed char)1) != G.lev + 27) eblk.push_back((int)b);
         if (any) xblk.push_back((int)b);
         else pure.push_back((int)b);
     }
@@ -578,6 +581,10 @@ void build_smr(kr_ctx *c, std::vector<BlockGeo> &g) {
     c->d_xblk = dalloc<int>(xblk.size());
     if (!xblk.empty())
         KR_HIP(hipMemcpy(c->d_xblk, xblk.data(), xblk.size() * sizeof(int), hipMemcpyHostToDevice));
+    c->neblk = (int)eblk.size();
+    c->d_eblk = dalloc<int>(eblk.size());
+    if (!eblk.empty())
+        KR_HIP(hipMemcpy(c->d_eblk, eblk.data(), eblk.size() * sizeof(int), hipMemcpyHostToDevice));
     c->npure = (int)pure.size();
     c->d_pure = dalloc<int>(pure.size());
     if (!pure.empty())
@@ -1173,7 +1180,7 @@ struct Launcher {
             // shared edges, flux restriction on the faces whose neighbour is
             // finer), then the update with the finer side's EMF write-back and
             // intg_flx folded in
-            const int nx = MHD ? c->nxblk : 0;      // blocks whose edges a finer one shares
+            const int nx = MHD ? c->neblk : 0;      // blocks whose edges a finer one shares
             if (nx + c->nftask) {
                 // largest face side; one row covers an edge box (MHD) or at
                 // least one face side, tpr face tasks per row
@@ -1186,7 +1193,7 @@ struct Launcher {
                 run(MHD ? KR_K_EMF : KR_K_UPDATE, [&] {
                     hipLaunchKernelGGL((k_smr_restrict<FT, NV>), dim3(w / kSmrThreads, nx + frows),
                                        dim3(kSmrThreads), 0, c->stream, m, c->sv,
-                                       (const int *)c->d_xblk, nx, (const int2 *)c->d_ftask,
+                                       (const int *)c->d_eblk, nx, (const int2 *)c->d_ftask,
                                        c->nftask, fmax, tpr);
                 });
             }

@@ -289,19 +289,21 @@ __device__ __forceinline__ FT smr_edge_read(const MeshView<FT> &m, const BlockGe
 }
 
 // act_flx of a stage in one launch: rows below nx restrict the EMFs of the
-// coarser blocks' shared edges (block xblk[row], one thread per edge-box
+// coarser blocks' shared edges (block eblk[row], one thread per edge-box
 // point), the others restrict the fluxes of the faces whose neighbour is
 // finer, tpr tasks per row (ftask[(row - nx) * tpr + k], fmax threads per
 // task).  Both read only what the sweep wrote and write disjoint coarser
-// data.
+// data.  Only
+// blocks that touch a finer level have rows (all cross-level blocks, mixed,
+// 442 blocks of 16^3: 33.9 us; these: 26.9).
 template <class FT, int NV>
 __global__ void __launch_bounds__(kSmrThreads) k_smr_restrict(MeshView<FT> m, SmrView s,
-                                                             const int *xblk, int nx,
+                                                             const int *eblk, int nx,
                                                              const int2 *ftask, int ntask,
                                                              int fmax, int tpr) {
     const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if ((int)blockIdx.y < nx) {
-        if constexpr (NV == 8) smr_emf_coarse_at(m, s, xblk[blockIdx.y], t);
+        if constexpr (NV == 8) smr_emf_coarse_at(m, s, eblk[blockIdx.y], t);
     } else {
         const int k = (int)(t / fmax);
         const int task = ((int)blockIdx.y - nx) * tpr + k;
