@@ -882,8 +882,15 @@ void commit(kr_ctx *c) {
     }
     // cell-centred E for the staged EMF kernel, when it runs
     const bool may_stage = !c->fused || kSweepVariants[c->candidates.back()].kernel == SK_STAGED;
-    if (c->mhd && !c->plane && (may_stage || (c->smr && c->prod < 0)))
+    if (c->mhd && !c->plane && (!c->fused || (c->smr && c->prod < 0))) {
         KR_HIP(hipMalloc(&c->EC, nb * 3 * c->ncell * fs));
+    } else if (c->mhd && !c->plane && may_stage &&
+               hipMalloc(&c->EC, nb * 3 * c->ncell * fs) != hipSuccess) {
+        // the tuner's candidate does without where memory ends: k_emf then
+        // forms the same products from W
+        (void)hipGetLastError();
+        c->EC = nullptr;
+    }
     c->stats.n_blocks = (int)nb;
     c->stats.n_cells = (long long)(nb * c->ncell);
     // 5 state passes per Heun cycle of (5 conserved + 3 face-B) FP64 values
