@@ -564,7 +564,8 @@ def main():
         if fused and dom == "update" and r.get("sweep_kernel"):
             kname = f"k_sweep_mx<{tl[0]},{tl[1]},{tl[2]}>"
         elif fused and dom == "update":
-            kname = f"k_sweep<{'float' if head == 'mixed' else 'double'},{tl[0]},{tl[1]},{tl[2]},{tl[3]}>"
+            kname = (f"k_sweep<{tl[0]},{tl[1]},{tl[2]},{tl[3]}>" if head == "mixed"
+                     else f"k_march<double,{tl[0]},{tl[1]},{tl[2]}>")
         else:
             kname = f"k_{dom}"
         cp = committed_profile(kname, workload)

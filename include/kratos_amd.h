@@ -114,7 +114,8 @@ typedef struct kr_stats {
     long long kernel_calls[8];
     double alg_bytes_per_cell_update;  /* algorithmic HBM bytes            */
     int    sweep_tile[4];  /* fused kernel in use: tile x, y, threads, waves
-                              per SIMD asked (zeros: staged path)           */
+                              per SIMD asked (zeros: the staged kernels, or
+                              the one-launch stage of 2-D and 1-D meshes)  */
     float  tune_ms[16];    /* autotuner: mean stage-kernel time per variant
                               over its tuning cycle (0: not timed)          */
     int    tune_pending;   /* variants the autotuner has still to time: the
@@ -122,8 +123,8 @@ typedef struct kr_stats {
                               variant each                                  */
     int    graph_ready;    /* 1 once the cycle's hipGraph is instantiated
                               (kr_advance then only replays it)            */
-    int    sweep_kernel;   /* the fused MHD kernel in use: 0 k_sweep, 1 the
-                              mixed form's k_sweep_mx                       */
+    int    sweep_kernel;   /* 1: the mixed MHD kernel k_sweep_mx is in use,
+                              0: another kernel                            */
 } kr_stats;
 
 enum kr_kernel_kind {
@@ -131,7 +132,8 @@ enum kr_kernel_kind {
     KR_K_FLUX_Z = 4, KR_K_EMF = 5, KR_K_UPDATE = 6, KR_K_BEGIN = 7
 };
 /* In the fused path the whole flux / EMF / update / CT stage is one launch,
- * reported under KR_K_UPDATE.                                             */
+ * reported under KR_K_UPDATE.  Small meshes take dt inside KR_K_C2P and launch
+ * neither KR_K_DTFIN nor KR_K_BEGIN.                                       */
 
 typedef struct kr_ctx kr_ctx;
 

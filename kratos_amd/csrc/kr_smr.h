@@ -293,9 +293,8 @@ __device__ __forceinline__ FT smr_edge_read(const MeshView<FT> &m, const BlockGe
 // point), the others restrict the fluxes of the faces whose neighbour is
 // finer, tpr tasks per row (ftask[(row - nx) * tpr + k], fmax threads per
 // task).  Both read only what the sweep wrote and write disjoint coarser
-// data.  Only
-// blocks that touch a finer level have rows (all cross-level blocks, mixed,
-// 442 blocks of 16^3: 33.9 us; these: 26.9).
+// data.  Only blocks that touch a finer level have rows (mixed, 442 blocks of
+// 16^3: 33.9 us with a row for every cross-level block, 26.9 so).
 template <class FT, int NV>
 __global__ void __launch_bounds__(kSmrThreads) k_smr_restrict(MeshView<FT> m, SmrView s,
                                                              const int *eblk, int nx,
