@@ -11,10 +11,20 @@
 // and everything up to r depends on the denominator alone, so quotients over
 // one denominator share it (hlld has 12 denominators), and 1 / (gamma - 1)
 // and its inverse come from the host.  Leaving out the scaling changes no
-// bit while n is 0 or within 2^-960 .. 2^500, d within 2^-200 .. 2^200 and
-// the quotient is normal; inputs that could leave that range (a velocity or
-// field below 2^-511 but not 0, any input above 2^60 or not a number, rho or p
-// below 2^-60) take the general function, a branch of the whole wave.
+// bit of a quotient while n is 0 or within 2^-968 .. 2^500 (below, the
+// remainder n - d q needs bits under 2^-1074), d within 2^-240 .. 2^240 and
+// the quotient is normal.  Inputs take the general function, a branch of the
+// whole wave, when a velocity or field is below 2^-840 but not 0, an input is
+// above 2^60 or not a number, or rho or p is below 2^-60.  Past that guard:
+//   - numerators linear in a transverse velocity or in the field keep the
+//     range.  The smallest are b_x (u* - u) in a star state and rho* v* in a
+//     double star; u* - u, or the rotation that makes v* from a v = 0, is at
+//     least 2^-53 of a wave speed above 2^-61, and rho* above 2^-62;
+//   - numerators of second order (b_x^2, b_t^2, rho* v.b, b_x rho* u* + m.b)
+//     may leave it, or vanish.  Their quotients are right to far better than
+//     2^-900, and each ends in a sum with one that is exact and at least
+//     2^-180: c_s^2 in both arguments of the speed's square roots, (s - u) e
+//     and e* in the energies.  What is off lies below half an ulp of the sum.
 //
 // The branches of hlld<double> (flat slopes, degenerate star states, the
 // region of the Riemann fan) become selects: with two waves on a SIMD the
@@ -82,11 +92,12 @@ __device__ __forceinline__ void plm_inc64(const double *lo, const double *hi, do
     }
 }
 
-// Smallest |value| among nonzero arguments, as an ordered integer of the
-// high word (0: largest); |x| >= 2^-900 <=> the integer >= kSmall64.
-constexpr unsigned kSmall64 = ((1023u - 900u) << 21) - 1u;
+// |x| as an ordered integer, its high word, with 0 the largest: the value
+// is at least kSmall64 <=> x = 0 or |x| > 2^-840.  The shift takes in the low
+// word: a subnormal below 2^-1042 has no other bits.
+constexpr unsigned kSmall64 = (1023u - 840u) << 21;
 __device__ __forceinline__ unsigned mag64(double x) {
-    return ((unsigned)__double2hiint(x) << 1) - 1u;
+    return (unsigned)((((unsigned long long)__double_as_longlong(x) << 1) - 1u) >> 32);
 }
 __device__ __forceinline__ unsigned umin3(unsigned a, unsigned b, unsigned c) {
     const unsigned d = a < b ? a : b;
