@@ -116,8 +116,17 @@ typedef struct kr_stats {
     int    sweep_tile[4];  /* fused kernel in use: tile x, y, threads, waves
                               per SIMD asked (zeros: the staged kernels, or
                               the one-launch stage of 2-D and 1-D meshes)  */
-    float  tune_ms[16];    /* autotuner: mean stage-kernel time per variant
-                              over its tuning cycle (0: not timed)          */
+    float  tune_ms[16];    /* autotuner: mean time of a stage past c2p per
+                              variant, over its tuning cycle (0: not timed).
+                              Entry by tile/threads (/waves): hydro, and mixed
+                              MHD with physical sides or on blocks that 8x8
+                              does not divide: 0 32x8/512, 1 32x8/512/4,
+                              2 16x16/512, 3 16x16/512/4, 4 16x8/256,
+                              5 8x8/192, 6 16x8/256/4; other mixed MHD:
+                              7 16x8/256, 8 32x8/512, 9 16x16/512, 10 8x8/192;
+                              FP64 MHD: 11 32x8/512, 12 16x8/512, 13 16x8/256,
+                              14 8x8/320, 15 16x16/512, 5 8x8/192; the staged
+                              kernels, where they are timed: 6              */
     int    tune_pending;   /* variants the autotuner has still to time: the
                               next that many cycles run eagerly, one
                               variant each                                  */

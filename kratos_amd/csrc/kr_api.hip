@@ -211,6 +211,7 @@ enum SweepKernel {
 };
 struct SweepVariant {
     int tx, ty, nt, waves, kernel;
+    int entry;      // of kr_stats.tune_ms: no two variants of one mesh share one
 };
 // k_march: a 16x8 tile's solves of a plane fill 256 threads twice or 512
 // once.  Two workgroups of 256 overlap on a compute unit and win where the
@@ -219,13 +220,13 @@ struct SweepVariant {
 // against 112 us).  Likewise 8x8 with 320 threads (one round; 32^3 cells in
 // 16^3 blocks: 36 against 46 us) and 192 (two; 128^3: 0.94 against 1.17 ms).
 constexpr SweepVariant kSweepVariants[] = {
-    {32, 8, 512, 1, SK_SWEEP},  {32, 8, 512, 4, SK_SWEEP}, {16, 16, 512, 1, SK_SWEEP},
-    {16, 16, 512, 4, SK_SWEEP}, {16, 8, 256, 1, SK_SWEEP}, {8, 8, 192, 1, SK_SWEEP},
-    {16, 8, 256, 4, SK_SWEEP},  {16, 8, 256, 1, SK_MX},    {32, 8, 512, 1, SK_MX},
-    {16, 16, 512, 1, SK_MX},    {8, 8, 192, 1, SK_MX},     {32, 8, 512, 1, SK_64},
-    {16, 8, 512, 1, SK_64},     {16, 8, 256, 1, SK_64},    {8, 8, 320, 1, SK_64},
-    {16, 16, 512, 1, SK_64_TILE}, {8, 8, 192, 1, SK_64_NARROW},
-    {16, 8, 256, 1, SK_ODD},    {8, 8, 192, 1, SK_ODD},   {0, 0, 0, 1, SK_STAGED},
+    {32, 8, 512, 1, SK_SWEEP, 0},    {32, 8, 512, 4, SK_SWEEP, 1},    {16, 16, 512, 1, SK_SWEEP, 2},
+    {16, 16, 512, 4, SK_SWEEP, 3},   {16, 8, 256, 1, SK_SWEEP, 4},    {8, 8, 192, 1, SK_SWEEP, 5},
+    {16, 8, 256, 4, SK_SWEEP, 6},    {16, 8, 256, 1, SK_MX, 7},       {32, 8, 512, 1, SK_MX, 8},
+    {16, 16, 512, 1, SK_MX, 9},      {8, 8, 192, 1, SK_MX, 10},       {32, 8, 512, 1, SK_64, 11},
+    {16, 8, 512, 1, SK_64, 12},      {16, 8, 256, 1, SK_64, 13},      {8, 8, 320, 1, SK_64, 14},
+    {16, 16, 512, 1, SK_64_TILE, 15}, {8, 8, 192, 1, SK_64_NARROW, 5}, {16, 8, 256, 1, SK_ODD, 4},
+    {8, 8, 192, 1, SK_ODD, 5},       {0, 0, 0, 1, SK_STAGED, 6},
 };
 constexpr int kNumSweepVariants = sizeof(kSweepVariants) / sizeof(kSweepVariants[0]);
 
@@ -1251,12 +1252,12 @@ void fill_tile_stats(kr_ctx *c) {
     c->stats.sweep_tile[2] = sv.nt;
     c->stats.sweep_tile[3] = sv.waves;
     c->stats.sweep_kernel = sv.kernel == SK_MX;
-    for (int v = 0; v < kNumSweepVariants && v < 16; ++v) c->stats.tune_ms[v] = c->tune_ms[v];
+    for (int v : c->candidates) c->stats.tune_ms[kSweepVariants[v].entry] = c->tune_ms[v];
 }
 
 // Tile autotuner on real cycles: while candidates are left, each cycle runs
-// the next candidate with events around its two stage-kernel launches; when
-// all are timed the fastest is kept.  Every variant performs the same
+// the next candidate with events around both its stages past c2p; when all
+// are timed the fastest is kept.  Every variant performs the same
 // arithmetic per face and per cell in the same order, so tuning cycles leave
 // exactly the state any fixed choice would.
 bool tuning(const kr_ctx *c) { return c->fused && !c->tuned; }
