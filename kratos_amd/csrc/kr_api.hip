@@ -1246,13 +1246,14 @@ void fill_tile_stats(kr_ctx *c) {
     c->stats.tune_pending = (c->fused && !c->tuned) ? (int)c->candidates.size() - c->tune_next : 0;
     c->stats.graph_ready = c->graph != nullptr;
     if (!c->fused) return;
+    for (int v : c->candidates) c->stats.tune_ms[kSweepVariants[v].entry] = c->tune_ms[v];
+    if (!c->fused_now()) return;
     const SweepVariant &sv = kSweepVariants[c->variant];
     c->stats.sweep_tile[0] = sv.tx;
     c->stats.sweep_tile[1] = sv.ty;
     c->stats.sweep_tile[2] = sv.nt;
     c->stats.sweep_tile[3] = sv.waves;
     c->stats.sweep_kernel = sv.kernel == SK_MX;
-    for (int v : c->candidates) c->stats.tune_ms[kSweepVariants[v].entry] = c->tune_ms[v];
 }
 
 // Tile autotuner on real cycles: while candidates are left, each cycle runs

@@ -46,5 +46,6 @@ def test_every_timed_variant_is_reported(gpu_lib, mhd, precision, blk, levels):
     assert timed.size == cand, (cand, st["tune_ms"])
     best = timed[np.argmin(ms[timed])]
     kept = st["sweep_tile"]
+    assert kept[0] > 0 or kept == (0, 0, 0, 0), kept      # zeros: the staged kernels
     if kept in ENTRY:
         assert best in ENTRY[kept], (kept, st["tune_ms"])
