@@ -75,8 +75,11 @@ __global__ void __launch_bounds__(NT) k_plane(MeshView<FT> m, int step) {
                 const CellSrc c = cell_src<FT, NV>(m, b, p);
                 double cons[5], prim[5], bc[3], bc_2[3], b_max[3];
                 bool heal_rho, moved;
-                cell_c2p<FT, MHD>(m, c.blk, step, cidx(m.n, c.p[0], c.p[1], c.p[2]), c.p[0], c.p[1], c.p[2], cons,
-                                  prim, bc, bc_2, b_max, heal_rho, moved);
+                const double *U = m.U + ((size_t)c.blk * 2 + step) * 5 * nc + cidx(m.n, c.p[0], c.p[1], c.p[2]);
+#pragma unroll
+                for (int v = 0; v < 5; ++v) cons[v] = U[(size_t)v * nc];
+                cell_c2p<FT, MHD>(m, c.blk, step, c.p[0], c.p[1], c.p[2], cons, prim, bc, bc_2, b_max,
+                                  heal_rho, moved);
 #pragma unroll
                 for (int v = 0; v < 5; ++v) w[v] = (FT)prim[v];
                 if constexpr (MHD) {

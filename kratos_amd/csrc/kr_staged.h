@@ -263,23 +263,17 @@ __device__ __forceinline__ double block_min(double v) {
 }
 
 // ------------------------------------------------------------------- c2p
-// Primitives of cell c = (i, j, k) of block b (hydro/eos/adiabatic.h:211-259,
-// mhd/eos/adiabatic.h:127-235) from its conserved state in slot `slot`: healed
-// values in cons, prim, for MHD the cell-centred B from the face average and
-// the squares and face maxima that the CFL speeds use.  heal_rho: rho was
-// raised to its floor; moved: the energy that the slot should hold differs
-// from what it holds (the subtract / add round trip of the magnetic part, or a
-// healed pressure).  Returns c_s^2.  The index c comes with i, j, k: k_c2p has
-// it before the 64-bit divisions that give them, so the state's loads don't
-// wait for those, and hydro, which needs no i, j, k, has no divisions (256^3
-// hydro: 0.180 -> 0.172 ms a launch mixed, 0.226 -> 0.222 FP64).
+// Primitives of cell (i, j, k) of block b (hydro/eos/adiabatic.h:211-259,
+// mhd/eos/adiabatic.h:127-235) from its conserved state in slot `slot`, which
+// the caller has loaded into cons: healed values in cons, prim, for MHD the
+// cell-centred B from the face average and the squares and face maxima that
+// the CFL speeds use.  heal_rho: rho was raised to its floor; moved: the energy
+// that the slot should hold differs from what it holds (the subtract / add
+// round trip of the magnetic part, or a healed pressure).  Returns c_s^2.
 template <class FT, bool MHD>
-__device__ __forceinline__ double cell_c2p(const MeshView<FT> &m, int b, int slot, size_t c, int i, int j,
-                                           int k, double *cons, double *prim, double *bc, double *bc_2,
+__device__ __forceinline__ double cell_c2p(const MeshView<FT> &m, int b, int slot, int i, int j, int k,
+                                           double *cons, double *prim, double *bc, double *bc_2,
                                            double *b_max, bool &heal_rho, bool &moved) {
-    const double *U = m.U + ((size_t)b * 2 + slot) * 5 * m.ncell + c;
-#pragma unroll
-    for (int v = 0; v < 5; ++v) cons[v] = U[(size_t)v * m.ncell];
     const EosPar e{m.gamma, m.cfl, m.d_floor, m.t_floor};
     if constexpr (MHD) {
         const double *BF = m.BF + ((size_t)b * 2 + slot) * 3 * m.nface;
@@ -348,13 +342,19 @@ __global__ void __launch_bounds__(kThreads) k_c2p(MeshView<FT> m, int step, cons
     const size_t c = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     double dtc = (double)FLT_MAX;
     if (c < m.ncell && !skip) {
+        // loaded before the 64-bit divisions that give i, j, k, which hydro does
+        // not need (128^3 MHD, a launch: with the loads after them 47.2 us mixed
+        // and 56.4 FP64, so 44.6 and 54.8; 256^3 hydro mixed with and without
+        // the divisions 180 and 171)
+        double *U = m.U + ((size_t)b * 2 + step) * 5 * m.ncell + c;
+        double cons[5], prim[5], bc[3], bc_2[3], b_max[3];
+#pragma unroll
+        for (int v = 0; v < 5; ++v) cons[v] = U[(size_t)v * m.ncell];
         const int i = (int)(c % m.n[0]);
         const int j = (int)((c / m.n[0]) % m.n[1]);
         const int k = (int)(c / ((size_t)m.n[0] * m.n[1]));
-        double cons[5], prim[5], bc[3], bc_2[3], b_max[3];
         bool heal_rho, moved;
-        const double cs2 = cell_c2p<FT, MHD>(m, b, step, c, i, j, k, cons, prim, bc, bc_2, b_max, heal_rho, moved);
-        double *U = m.U + ((size_t)b * 2 + step) * 5 * m.ncell + c;
+        const double cs2 = cell_c2p<FT, MHD>(m, b, step, i, j, k, cons, prim, bc, bc_2, b_max, heal_rho, moved);
         const BlockGeo &g = m.geo[b];
         FT *W = m.W + (size_t)b * NV * m.ncell + c;
         // the slot is written only where it does not hold the value already
