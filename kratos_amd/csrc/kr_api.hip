@@ -599,17 +599,19 @@ void build_smr(kr_ctx *c, std::vector<BlockGeo> &g) {
 
 HostShape host_shape(const kr_ctx *c, bool bf) {
     HostShape h{};
-    size_t nf = 1;
     for (int a = 0; a < 3; ++a) {
         h.n[a] = c->n[a];
         // n + (n > 1) faces per axis plus two ghost layers each side
         // (mhd/types/fld_data.cpp:18-26); a thin axis has one
         h.N[a] = c->n[a] + (c->n[a] > 1) + 4;
-        nf *= (size_t)h.N[a];
     }
     h.nvar = c->mhd ? 8 : 5;
     h.nu = c->ncell * h.nvar;
-    h.nbf = bf ? nf * 3 : 0;
+    auto at = [&](int x, int y, int z) { return (((size_t)z * h.N[1] + y) * h.N[0] + x) * 3; };
+    if (bf) {
+        h.bf0 = at(2, 2, 2);
+        h.nbf = at(h.N[0] - 3, h.N[1] - 3, h.N[2] - 3) + 3 - h.bf0;
+    }
     return h;
 }
 
@@ -1361,13 +1363,14 @@ double *noalloc_scratch() {
 
 namespace {
 
-// [i0, i0 + count) of the host arrays (u, then bf) against one buffer.
+// [i0, i0 + count) of what is moved of the host arrays (u, then bf) against
+// one buffer.
 template <class F> void each_part(const HostShape &h, size_t i0, size_t count, F &&f) {
     const size_t i1 = i0 + count;
     if (i0 < h.nu) f(false, i0, std::min(i1, h.nu) - i0, (size_t)0);
     if (i1 > h.nu) {
         const size_t k = std::max(i0, h.nu);
-        f(true, k - h.nu, i1 - k, k - i0);
+        f(true, k - h.nu + h.bf0, i1 - k, k - i0);
     }
 }
 
@@ -1430,6 +1433,11 @@ void download_one(kr_ctx *c, size_t b, double *u_aos, double *bf_aos) {
         [&](size_t i0, size_t cnt, double *buf) {
             hipLaunchKernelGGL(k_pack, dim3(ceil_div(cnt, kThreads)), dim3(kThreads), 0, c->stream, h, U,
                                BF, c->ncell, c->nface, i0, cnt, buf);
+            if (i0 == 0 && h.nbf) {         // the ghost layers that are not moved
+                const size_t end = h.bf0 + h.nbf, all = (size_t)h.N[0] * h.N[1] * h.N[2] * 3;
+                std::memset(bf_aos, 0, h.bf0 * sizeof(double));
+                std::memset(bf_aos + end, 0, (all - end) * sizeof(double));
+            }
         },
         [&](size_t i0, size_t cnt, const double *buf) {
             each_part(h, i0, cnt, [&](bool bf, size_t at, size_t n, size_t off) {

@@ -15,14 +15,18 @@
 namespace kr {
 
 // Host arrays of a block: u (ncell * nvar), then for MHD the face array with
-// two ghost layers a side, N[a] = n[a] + (n[a] > 1) + 4.
+// two ghost layers a side, N[a] = n[a] + (n[a] > 1) + 4.  Of that one the
+// doubles from the block's first face to its last are moved, bf0 .. bf0 + nbf:
+// the ghost layers before and behind are not read, and zeros on the way back
+// (four fifths of a 2-D block's array, 24 of 25 rows of a 1-D block's).
 struct HostShape {
     int n[3], N[3], nvar;
-    size_t nu, nbf;          // doubles of u and of bf
+    size_t nu, bf0, nbf;     // doubles of u, first and number of those of bf
 };
 
-// Doubles [i0, i0 + count) of a block's host arrays (u, then bf) into out,
-// from slot 0: u's cell-centred B is the face average, ghost faces are 0.
+// Doubles [i0, i0 + count) of what is moved of a block's host arrays (u, then
+// bf) into out, from slot 0: u's cell-centred B is the face average, ghost
+// faces are 0.
 __global__ void __launch_bounds__(kThreads) k_pack(HostShape h, const double *U, const double *BF,
                                                    size_t ncell, size_t nface, size_t i0, size_t count,
                                                    double *out) {
@@ -46,7 +50,7 @@ __global__ void __launch_bounds__(kThreads) k_pack(HostShape h, const double *U,
             v = (f[0] + f[sh]) / 2;
         }
     } else {
-        const size_t j = i - h.nu;
+        const size_t j = i - h.nu + h.bf0;
         const unsigned f = (unsigned)(j / 3);
         const int a = (int)(j - (size_t)f * 3);
         const int x = (int)(f % h.N[0]) - 2, y = (int)(f / h.N[0] % h.N[1]) - 2,
@@ -69,7 +73,7 @@ __global__ void __launch_bounds__(kThreads) k_unpack(HostShape h, double *U, dou
         const int k = (int)(i - (size_t)c * h.nvar);
         if (k < 5) U[(size_t)k * ncell + c] = in[t];
     } else {
-        const size_t j = i - h.nu;
+        const size_t j = i - h.nu + h.bf0;
         const unsigned f = (unsigned)(j / 3);
         const int a = (int)(j - (size_t)f * 3);
         const int x = (int)(f % h.N[0]) - 2, y = (int)(f / h.N[0] % h.N[1]) - 2,
