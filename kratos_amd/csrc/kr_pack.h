@@ -7,7 +7,8 @@
 // two vectors and three strided loops over each block (128 MHD blocks of 8^3:
 // 35 us a block).  Here one thread moves one double of the host arrays, with
 // consecutive threads on consecutive doubles, so the bus sees full lines;
-// what is left on the host is one contiguous copy per array.
+// what is left on the host is one contiguous copy per array.  (Small hydro
+// blocks, one range and no faces, are transposed on the host: kr_api.hip.)
 #pragma once
 
 #include "kr_staged.h"
