@@ -315,6 +315,8 @@ struct kr_ctx {
     double *d_in = nullptr;         // device copy of the halves, for large uploads
     hipEvent_t pin_ev[2] = {nullptr, nullptr};
 
+    // k_emf runs whatever the tuner chooses
+    bool needs_ec() const { return mhd && !plane && (!fused || (smr && prod < 0)); }
     // the fused kernels run (or, while tuning, the candidate at hand is one)
     bool fused_now() const { return fused && kSweepVariants[variant].kernel != SK_STAGED; }
 
@@ -340,7 +342,7 @@ struct kr_ctx {
         m.W = (FT *)W;
         for (int a = 0; a < 3; ++a) m.F[a] = (FT *)F[a];
         m.EE = (FT *)EE;
-        m.EC = !fused_now() || (smr && prod < 0) ? (FT *)EC : nullptr;
+        m.EC = !fused_now() || needs_ec() ? (FT *)EC : nullptr;
         m.geo = geo;
         m.ts = ts;
         m.dt_part = dt_part;
@@ -873,7 +875,6 @@ void commit(kr_ctx *c) {
     c->n_red_part = c->n_dt_part;
     c->red_part = dalloc<double>(c->n_red_part);
     c->red_out = dalloc<double>(1);
-    // cell-centred E for the staged EMF (c2p writes it only when allocated)
     // producer form of the fused kernel for the blocks of a refined mesh
     // that touch another level: 16x8 or 8x8 column tiles
     c->prod = -1;
@@ -891,16 +892,17 @@ void commit(kr_ctx *c) {
         c->tuned = true;
         c->tune_next = 0;
     }
-    // cell-centred E for the staged EMF kernel, when it runs
-    const bool may_stage = !c->fused || kSweepVariants[c->candidates.back()].kernel == SK_STAGED;
-    if (c->mhd && !c->plane && (!c->fused || (c->smr && c->prod < 0))) {
+    // cell-centred E for the staged EMF kernel, when it runs; tune_cycle gives
+    // the array back if the staged kernels are a candidate and lose
+    if (c->needs_ec()) {
         KR_HIP(hipMalloc(&c->EC, nb * 3 * c->ncell * fs));
-    } else if (c->mhd && !c->plane && may_stage &&
+    } else if (c->mhd && c->fused && kSweepVariants[c->candidates.back()].kernel == SK_STAGED &&
                hipMalloc(&c->EC, nb * 3 * c->ncell * fs) != hipSuccess) {
-        // the tuner's candidate does without where memory ends: k_emf then
-        // forms the same products from W
+        // memory ends here: the mesh runs without that candidate
         (void)hipGetLastError();
         c->EC = nullptr;
+        c->candidates.pop_back();
+        c->tuned = c->candidates.size() <= 1;
     }
     c->stats.n_blocks = (int)nb;
     c->stats.n_cells = (long long)(nb * c->ncell);
@@ -1294,6 +1296,10 @@ void tune_cycle(kr_ctx *c) {
             if (c->tune_ms[w] < c->tune_ms[pick]) pick = w;
         c->variant = pick;
         c->tuned = true;
+        if (c->EC && c->fused_now() && !c->needs_ec()) {
+            (void)hipFree(c->EC);
+            c->EC = nullptr;
+        }
     }
 }
 

@@ -525,13 +525,8 @@ __device__ __forceinline__ FT ec_at(const MeshView<FT> &m, int b, const int *p, 
     bool in = true;
 #pragma unroll
     for (int a = 0; a < 3; ++a) in &= p[a] >= 0 && p[a] < m.n[a];
-    if (in) {   // the block's own cell: the c2p value (equal to B x v of its w)
-        const size_t c = cidx(m.n, p[0], p[1], p[2]);
-        if (m.EC) return m.EC[((size_t)b * 3 + ax[0]) * m.ncell + c];
-        const FT *W = m.W + (size_t)b * 8 * m.ncell + c;
-        const size_t s = m.ncell;
-        return W[(BCC + ax[1]) * s] * W[(MOM + ax[2]) * s] - W[(BCC + ax[2]) * s] * W[(MOM + ax[1]) * s];
-    }
+    if (in)     // the block's own cell: the c2p value (equal to B x v of its w)
+        return m.EC[((size_t)b * 3 + ax[0]) * m.ncell + cidx(m.n, p[0], p[1], p[2])];
     FT w[8];
     load_cell<FT, 8>(m, b, p, w);
     return w[BCC + ax[1]] * w[MOM + ax[2]] - w[BCC + ax[2]] * w[MOM + ax[1]];
