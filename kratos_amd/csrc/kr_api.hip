@@ -960,20 +960,26 @@ struct Launcher {
         const unsigned kz = ranges(fn, variant, threads, nt, nb, lat);
         hipLaunchKernelGGL(fn, dim3(nt, nb, kz), dim3(threads), 0, c->stream, m, step);
     }
+    // the builds with the rules of physical sides serve one-level meshes only
+    // (npfill); the producer forms are for refined ones
     template <int TX, int TY, int NT, int W, int PROD = 0>
     void sweep_t(const MeshView<float> &m, int step, unsigned nb) {
-        // npfill: physical sides (one-level meshes only)
-        launch(c->npfill ? k_sweep<TX, TY, NT, W, PROD, true> : k_sweep<TX, TY, NT, W, PROD, false>, m,
-               step, PROD ? kNumSweepVariants : c->variant, TX, TY, NT, nb, kLatMhdMixed);
+        auto fn = k_sweep<TX, TY, NT, W, PROD, false>;
+        if constexpr (PROD == 0)
+            if (c->npfill) fn = k_sweep<TX, TY, NT, W, PROD, true>;
+        launch(fn, m, step, PROD ? kNumSweepVariants : c->variant, TX, TY, NT, nb, kLatMhdMixed);
     }
     template <class FT, int TX, int TY, int NT, int PROD = 0>
     void march_t(const MeshView<FT> &m, int step, unsigned nb) {
-        // FP32: the build with the rules of physical sides everywhere (they do
-        // nothing on a periodic mesh): it rounds as the staged kernels do
-        launch(c->npfill || std::is_same_v<FT, float> ? k_march<FT, TX, TY, NT, PROD, true>
-                                                      : k_march<FT, TX, TY, NT, PROD, false>,
-               m, step, PROD ? kNumSweepVariants : c->variant, TX, TY, NT, nb,
-               std::is_same_v<FT, double> ? kLatMhd64 : kLatMhdMixed);
+        // FP32: always the build with the rules of physical sides (they do
+        // nothing on a periodic mesh): it rounds as the staged kernels do,
+        // between which and it the tuner chooses
+        constexpr bool f32 = std::is_same_v<FT, float>;
+        auto fn = k_march<FT, TX, TY, NT, PROD, f32>;
+        if constexpr (!f32 && PROD == 0)
+            if (c->npfill) fn = k_march<FT, TX, TY, NT, PROD, true>;
+        launch(fn, m, step, PROD ? kNumSweepVariants : c->variant, TX, TY, NT, nb,
+               f32 ? kLatMhdMixed : kLatMhd64);
     }
     // FP64: fluxes and edge EMFs of the listed blocks into F / EE (no update)
     void sweep_prod(const MeshView<double> &m, int step, unsigned nb) {
