@@ -981,7 +981,12 @@ struct Launcher {
         launch(fn, m, step, PROD ? kNumSweepVariants : c->variant, TX, TY, NT, nb,
                f32 ? kLatMhdMixed : kLatMhd64);
     }
-    // FP64: fluxes and edge EMFs of the listed blocks into F / EE (no update)
+    // FP64: fluxes and edge EMFs of the listed blocks into F / EE (no update).
+    // 8x8 tiles: 320 threads (one round of a plane's solves) while the tiles
+    // leave compute units idle, 192 (two) beyond.  A launch with 320 and with
+    // 192, blocks of 8^3: 112 workgroups 47 and 67 us, 448 140 and 138 to 144,
+    // 1,024 283 and 280, 1,840 569 and 522; of 24^3: 1,008 727 and 701, 4,032
+    // 2,896 and 2,607.
     void sweep_prod(const MeshView<double> &m, int step, unsigned nb) {
         if (c->prod == 0) march_t<double, 16, 8, 256, 1>(m, step, nb);
         else if (nb * (unsigned)((c->n[0] / 8) * (c->n[1] / 8)) <= 512) march_t<double, 8, 8, 320, 1>(m, step, nb);
