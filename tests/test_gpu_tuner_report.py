@@ -49,3 +49,20 @@ def test_every_timed_variant_is_reported(gpu_lib, mhd, precision, blk, levels):
     assert kept[0] > 0 or kept == (0, 0, 0, 0), kept      # zeros: the staged kernels
     if kept in ENTRY:
         assert best in ENTRY[kept], (kept, st["tune_ms"])
+
+
+@pytest.mark.parametrize("path,n,tile,entries", [
+    ("auto", 32, (8, 8, 0), [5, 14]), ("fused", 32, (8, 8, 0), [5, 14]), ("auto", 32, (16, 8, 0), [12, 13]),
+    ("fused", 24, (0, 0, 0), [5, 14])])
+def test_fp64_tile_times_both_thread_counts(gpu_lib, path, n, tile, entries):
+    """Where an FP64 MHD mesh runs one tile, asked for by kr_config.tile or the
+    only one that fits, both of its builds are timed."""
+    spec = kratos_amd.MeshSpec((2 * n, 2 * n, n), (n, n, n))
+    u, b, _ = problems.turbulence(spec.n_cell_global, seed=5)
+    ctx = kratos_amd.Context(spec, kratos_amd.Physics(mhd=True), "fp64", path=path, tile=tile)
+    ctx.upload(u, b)
+    ctx.advance(4)
+    st = ctx.stats()
+    ctx.close()
+    assert list(np.flatnonzero(st["tune_ms"])) == entries
+    assert st["sweep_tile"][:2] == (tile[:2] if tile[0] else (8, 8))
