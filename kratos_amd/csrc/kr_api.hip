@@ -837,7 +837,7 @@ void commit(kr_ctx *c) {
     c->U = dalloc<double>(nb * 2 * 5 * c->ncell);
     if (c->mhd) c->BF = dalloc<double>(nb * 2 * 3 * c->nface);
     KR_HIP(hipMalloc(&c->W, nw * c->nv * c->ncell * fs));
-    c->plane = c->ndim < 3 && c->cfg.kernel_path == KR_PATH_AUTO;
+    c->plane = c->ndim > 0 && c->ndim < 3 && c->cfg.kernel_path == KR_PATH_AUTO;
     for (int a = 0; a < c->ndim && !c->plane; ++a)
         KR_HIP(hipMalloc(&c->F[a], nb * c->nv * c->nfa[a] * fs));
     if (c->mhd && !c->plane) KR_HIP(hipMalloc(&c->EE, nb * 3 * c->nface * fs));
@@ -1198,10 +1198,11 @@ struct Launcher {
                 hipLaunchKernelGGL((k_flux<FT, MHD, 1>), dim3(ceil_div(c->nfa[1], kThreads), ns),
                                    blk, 0, c->stream, ms, step);
             });
-        run(KR_K_FLUX_X, [&] {
-            hipLaunchKernelGGL((k_flux<FT, MHD, 0>), dim3(ceil_div(c->nfa[0], kThreads), ns), blk,
-                               0, c->stream, ms, step);
-        });
+        if (c->ndim > 0)                    // a block of one cell has no sweep
+            run(KR_K_FLUX_X, [&] {
+                hipLaunchKernelGGL((k_flux<FT, MHD, 0>), dim3(ceil_div(c->nfa[0], kThreads), ns),
+                                   blk, 0, c->stream, ms, step);
+            });
         if constexpr (MHD)
             run(KR_K_EMF, [&] {
                 hipLaunchKernelGGL(k_emf<FT>, dim3(ceil_div(c->nface, kThreads), ns, 3), blk, 0,
