@@ -238,6 +238,14 @@ constexpr SweepVariant kSweepVariants[] = {
     {8, 8, 192, 1, SK_ODD, 5},       {0, 0, 0, 1, SK_STAGED, 6},
 };
 constexpr int kNumSweepVariants = sizeof(kSweepVariants) / sizeof(kSweepVariants[0]);
+// Index of a variant (a compile-time error if the table has none such).
+constexpr int variant_of(int kernel, int tx, int ty, int nt, int waves = 1) {
+    for (int v = 0; v < kNumSweepVariants; ++v) {
+        const SweepVariant &s = kSweepVariants[v];
+        if (s.kernel == kernel && s.tx == tx && s.ty == ty && s.nt == nt && s.waves == waves) return v;
+    }
+    throw std::logic_error("no such stage variant");
+}
 
 }  // namespace
 
@@ -891,7 +899,7 @@ void commit(kr_ctx *c) {
     // so the pure blocks take the producer's tile; no tuning.  The FP64 form
     // keeps two launches (the combined kernel would run at one wave per SIMD)
     if (c->prod >= 0 && c->mixed) {
-        const int want = c->prod == 0 ? 4 : 5;      // 16x8/256, 8x8/192
+        const int want = c->prod == 0 ? variant_of(SK_SWEEP, 16, 8, 256) : variant_of(SK_SWEEP, 8, 8, 192);
         c->candidates.assign(1, want);
         c->variant = want;
         c->tuned = true;
@@ -1010,39 +1018,42 @@ struct Launcher {
     // hydro: the one-wave-per-SIMD-minimum variants of the tile table
     template <class FT> void sweep_hyd(const MeshView<FT> &m, int step, int variant, unsigned nb) {
         switch (variant) {
-        case 0: sweep_hyd_t<FT, 32, 8, 512>(m, step, nb); break;
-        case 2: sweep_hyd_t<FT, 16, 16, 512>(m, step, nb); break;
-        case 5: sweep_hyd_t<FT, 8, 8, 192>(m, step, nb); break;
-        default: sweep_hyd_t<FT, 16, 8, 256>(m, step, nb); break;
+        case variant_of(SK_SWEEP, 32, 8, 512): sweep_hyd_t<FT, 32, 8, 512>(m, step, nb); break;
+        case variant_of(SK_SWEEP, 16, 16, 512): sweep_hyd_t<FT, 16, 16, 512>(m, step, nb); break;
+        case variant_of(SK_SWEEP, 16, 8, 256): sweep_hyd_t<FT, 16, 8, 256>(m, step, nb); break;
+        case variant_of(SK_SWEEP, 8, 8, 192): sweep_hyd_t<FT, 8, 8, 192>(m, step, nb); break;
+        default: throw std::logic_error("not a hydro variant");
         }
     }
 
     // grid rows: nb blocks (m.blist maps a row to its block when set)
     void sweep(const MeshView<float> &m, int step, int variant, unsigned nb) {
         switch (variant) {
-        case 0: sweep_t<32, 8, 512, 1>(m, step, nb); break;
-        case 1: sweep_t<32, 8, 512, 4>(m, step, nb); break;
-        case 2: sweep_t<16, 16, 512, 1>(m, step, nb); break;
-        case 3: sweep_t<16, 16, 512, 4>(m, step, nb); break;
-        case 4: sweep_t<16, 8, 256, 1>(m, step, nb); break;
-        case 5: sweep_t<8, 8, 192, 1>(m, step, nb); break;
-        case 6: sweep_t<16, 8, 256, 4>(m, step, nb); break;
-        case 7: sweep_mx_t<16, 8, 256>(m, step, nb); break;
-        case 8: sweep_mx_t<32, 8, 512>(m, step, nb); break;
-        case 9: sweep_mx_t<16, 16, 512>(m, step, nb); break;
-        case 10: sweep_mx_t<8, 8, 192>(m, step, nb); break;
-        case 17: march_t<float, 16, 8, 256>(m, step, nb); break;
-        default: march_t<float, 8, 8, 192>(m, step, nb); break;
+        case variant_of(SK_SWEEP, 32, 8, 512): sweep_t<32, 8, 512, 1>(m, step, nb); break;
+        case variant_of(SK_SWEEP, 32, 8, 512, 4): sweep_t<32, 8, 512, 4>(m, step, nb); break;
+        case variant_of(SK_SWEEP, 16, 16, 512): sweep_t<16, 16, 512, 1>(m, step, nb); break;
+        case variant_of(SK_SWEEP, 16, 16, 512, 4): sweep_t<16, 16, 512, 4>(m, step, nb); break;
+        case variant_of(SK_SWEEP, 16, 8, 256): sweep_t<16, 8, 256, 1>(m, step, nb); break;
+        case variant_of(SK_SWEEP, 16, 8, 256, 4): sweep_t<16, 8, 256, 4>(m, step, nb); break;
+        case variant_of(SK_SWEEP, 8, 8, 192): sweep_t<8, 8, 192, 1>(m, step, nb); break;
+        case variant_of(SK_MX, 16, 8, 256): sweep_mx_t<16, 8, 256>(m, step, nb); break;
+        case variant_of(SK_MX, 32, 8, 512): sweep_mx_t<32, 8, 512>(m, step, nb); break;
+        case variant_of(SK_MX, 16, 16, 512): sweep_mx_t<16, 16, 512>(m, step, nb); break;
+        case variant_of(SK_MX, 8, 8, 192): sweep_mx_t<8, 8, 192>(m, step, nb); break;
+        case variant_of(SK_ODD, 16, 8, 256): march_t<float, 16, 8, 256>(m, step, nb); break;
+        case variant_of(SK_ODD, 8, 8, 192): march_t<float, 8, 8, 192>(m, step, nb); break;
+        default: throw std::logic_error("not a mixed MHD variant");
         }
     }
     void sweep(const MeshView<double> &m, int step, int variant, unsigned nb) {
         switch (variant) {
-        case 11: march_t<double, 32, 8, 512>(m, step, nb); break;
-        case 12: march_t<double, 16, 8, 512>(m, step, nb); break;
-        case 13: march_t<double, 16, 8, 256>(m, step, nb); break;
-        case 14: march_t<double, 8, 8, 320>(m, step, nb); break;
-        case 15: march_t<double, 16, 16, 512>(m, step, nb); break;
-        default: march_t<double, 8, 8, 192>(m, step, nb); break;
+        case variant_of(SK_64, 32, 8, 512): march_t<double, 32, 8, 512>(m, step, nb); break;
+        case variant_of(SK_64, 16, 8, 512): march_t<double, 16, 8, 512>(m, step, nb); break;
+        case variant_of(SK_64, 16, 8, 256): march_t<double, 16, 8, 256>(m, step, nb); break;
+        case variant_of(SK_64, 8, 8, 320): march_t<double, 8, 8, 320>(m, step, nb); break;
+        case variant_of(SK_64_TILE, 16, 16, 512): march_t<double, 16, 16, 512>(m, step, nb); break;
+        case variant_of(SK_64_NARROW, 8, 8, 192): march_t<double, 8, 8, 192>(m, step, nb); break;
+        default: throw std::logic_error("not an FP64 MHD variant");
         }
     }
     // Ensembles: the cycle's work list (the tiles of the boxes still running,
