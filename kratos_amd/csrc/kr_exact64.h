@@ -113,7 +113,7 @@ struct Gam64 {
 template <class T> __device__ __forceinline__ T sel(bool c, T a, T b) { return c ? a : b; }
 
 // hlld<double> (mhd/riemann/hlld.h:81-298) without the normal slot BCC:
-// about 670 VALU instructions where the general function issues 1,000.
+// about 650 VALU instructions where the general function issues 1,000.
 __device__ __forceinline__ void hlld64(double *flx, const double *wl, const double *wr, const Gam64 &k) {
     {
         // the sum is not a number if one of them is
