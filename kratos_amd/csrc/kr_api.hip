@@ -188,6 +188,7 @@ static_assert(5 * kHostPackCells <= kPinDoubles, "a block fits one half of the b
 // and 112.9, 1,024 124.1 and 137.9; FP64 hydro: 54.1 and 51.4, 71.6 and 70.2,
 // 74.9 and 76.0, 89.6 and 97.6, 112.2 and 124.3.
 constexpr size_t kFinWorkgroups = 320;
+static_assert(kFinWorkgroups <= 64 * kFinWaves, "one CFL partial a thread of k_dt_finalize");
 
 // Most workgroups of a staged MHD update whose cells and three face families
 // are layers of the grid: above, one layer fills the GPU and a point's cell

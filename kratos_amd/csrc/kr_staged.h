@@ -331,6 +331,7 @@ __device__ __forceinline__ void take_dt(TimeState *ts, double cfl_dt) {
 // spent on either (k_cycle_begin and k_dt_finalize, together 6 to 9 us of a
 // cycle; on large meshes the arrivals would cost more than the launches).
 // arrived[g] counts the group's workgroups and is left at 0.
+constexpr int kFinWaves = 16;          // waves of k_dt_finalize
 template <class FT, bool MHD, bool FIN>
 __global__ void __launch_bounds__(kThreads) k_c2p(MeshView<FT> m, int step, const int *grp_first,
                                                   int *arrived) {
@@ -398,12 +399,25 @@ __global__ void __launch_bounds__(kThreads) k_c2p(MeshView<FT> m, int step, cons
         }
         __syncthreads();
         if (!s_last) return;
-        double v = (double)FLT_MAX;
-        for (size_t i = (size_t)first * gridDim.x + threadIdx.x; i < (size_t)last * gridDim.x; i += kThreads)
-            v = pmin(v, __hip_atomic_load(m.dt_part + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-        __syncthreads();                     // block_min's scratch is read above by thread 0
-        v = block_min(v);
+        // the partials in k_dt_finalize's order, 64 of them a wave's: pmin keeps
+        // or drops a NaN by its place, and a state that holds one is to take the
+        // same dt on either side of the line
+        __shared__ double s_min[kFinWaves];
+        const double *part = m.dt_part + (size_t)first * gridDim.x;
+        const int n = (last - first) * (int)gridDim.x, waves = (n + 63) / 64;
+        for (int w = threadIdx.x >> 6; w < waves; w += kThreads / 64) {
+            const int i = w * 64 + (threadIdx.x & 63);
+            double v = (double)FLT_MAX;
+            if (i < n) v = pmin(v, __hip_atomic_load(part + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) v = pmin(v, __shfl_xor(v, off, 64));
+            if ((threadIdx.x & 63) == 0) s_min[w] = v;
+        }
+        __syncthreads();
         if (threadIdx.x == 0) {
+            double v = s_min[0];
+            for (int w = 1; w < waves; ++w) v = pmin(v, s_min[w]);
+            if (waves < kFinWaves) v = pmin(v, (double)FLT_MAX);     // its idle waves
             ts->skip = skip ? 1 : 0;
             if (!skip) {
                 ts->cycles += 1;
